@@ -295,8 +295,8 @@ __global__ __launch_bounds__(256, 4) void k_s8n_gemm(const int8_t *__restrict__ 
   const int8_t *ap[2];
 #pragma unroll
   for (int t = 0; t < 2; t++) ap[t] = q + s_q[lr0 + 16 * t + (lane & 15)] + kc;
-  const int kmain = Kp & ~63;
-  const bool kin = kmain + kc < Kp;  // this lane's chunk of the last partial step holds k < Kp
+  const int kmain = Kp <= 64 ? 0 : Kp & ~63;  // the whole 64-wide steps before the last one (Kp 64: that one step)
+  const bool kin = kmain + kc < Kp;  // this lane's chunk of the last step holds k < Kp
   // one K step (Kp <= 64, the expansions): the A fragments once for every group
   v4i a1[2];
   if (Kp <= 64) {

@@ -249,6 +249,13 @@ def test_pw_s8_unaligned_output_rows(hip):
     assert pw_case(hip, 2, 7, 5, 40, 136, 1, opad=1, seed=13, ldo_extra=1)
 
 
+@pytest.mark.parametrize("K", [48, 49, 52, 64, 65, 128])
+def test_pw_s8_whole_k_steps(hip, K):
+    """Rows that end exactly with a 64-wide K step (Kp 64, 128) and beside it, with and without a residual"""
+    assert pw_case(hip, 2, 6, 11, K, 96, 1, seed=50 + K)
+    assert pw_case(hip, 2, 6, 11, K, 24, 0, res=True, seed=60 + K)
+
+
 def test_gemm_requant_config0(hip):
     H = hip
     rng = np.random.default_rng(2024)
