@@ -317,13 +317,14 @@ BNH_DEV v8h h8_v(H8 a) {
   return o;
 }
 
+// a block runs the tile rows of one strip that fall to its segment of nseg
 template <int NCH, int NCB, int ACT>  // NCH = Cp / 32 MFMA k steps, NCB = Kp / 16 output channel blocks
 __global__ __launch_bounds__(256, 2) void k_wino_f16r(const uint16_t *__restrict__ x, long long x_ws, int H, int W,
                                                       int C, int ldx, const uint16_t *__restrict__ U,
                                                       const float *__restrict__ bias, int K,
                                                       uint16_t *__restrict__ out, long long o_ws, int ldo, int opad,
                                                       const uint16_t *__restrict__ res, long long r_ws, int ldr,
-                                                      int rpad, int strips) {
+                                                      int rpad, int strips, int nseg) {
   constexpr int CP = 32 * NCH, KP = 16 * NCB, RING = 6;
   constexpr int XS = CP + 8;                 // ring pixel stride (halves)
   constexpr int XR = WT_COLS * XS;           // ring row stride (halves)
@@ -336,8 +337,10 @@ __global__ __launch_bounds__(256, 2) void k_wino_f16r(const uint16_t *__restrict
   __shared__ __attribute__((aligned(16))) float Bs[KP];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wi = __builtin_amdgcn_readfirstlane(tid >> 6);  // this wave's row of positions
-  const int win = blockIdx.x / strips, strip = blockIdx.x % strips;
-  const int T = W / 2, tx0 = strip * WT_TILES, Wp = W + 2, NS = H / 2, c8 = C / 8;
+  const int win = blockIdx.x / (strips * nseg), seg = blockIdx.x / strips % nseg, strip = blockIdx.x % strips;
+  const int T = W / 2, tx0 = strip * WT_TILES, Wp = W + 2, c8 = C / 8;
+  const int S0 = (int)((long long)(H / 2) * seg / nseg);        // this block's tile rows [S0, NS)
+  const int NS = (int)((long long)(H / 2) * (seg + 1) / nseg);
   const int ntl = T - tx0 < WT_TILES ? T - tx0 : WT_TILES;  // tiles of this strip that are stored
   // the window's haloed input as one buffer (columns past the image read the next row or zeros; tiles past T are
   // never stored)
@@ -382,11 +385,11 @@ __global__ __launch_bounds__(256, 2) void k_wino_f16r(const uint16_t *__restrict
     for (int i = tid; i < RING * XR / 8; i += 256) ((v4i *)Xs)[i] = (v4i){0, 0, 0, 0};
   for (int i = tid; i < KP; i += 256) Bs[i] = i < K ? bias[i] : 0.f;
   __syncthreads();
-  fetch(0);
+  fetch(2 * S0);
   commit(0);
-  fetch(2);
+  fetch(2 * S0 + 2);
   commit(2);
-  if (NS > 1) fetch(4);
+  if (S0 + 1 < NS) fetch(2 * S0 + 4);
   // the output and residual of the window as buffers: 32-bit byte offsets, a lane part and a scalar row part
   const __amdgpu_buffer_rsrc_t orr = __builtin_amdgcn_make_buffer_rsrc(
       (void *)(out + win * o_ws), 0, (int)((long long)(H + 2 * opad) * (W + 2 * opad) * ldo * 2), 0x00020000);
@@ -411,7 +414,7 @@ __global__ __launch_bounds__(256, 2) void k_wino_f16r(const uint16_t *__restrict
   auto steps = [&](auto add_rows) {
   constexpr bool ADD = decltype(add_rows)::value;
   int base = 0;  // ring row of the step's first input row
-  for (int s = 0; s < NS; s++) {
+  for (int s = S0; s < NS; s++) {
     // the rows of step s + 1 (loaded during step s - 1) into the ring slots step s - 1 read last
     if (s + 1 < NS) commit(base == 0 ? 4 : base - 2);
     if (s + 2 < NS) fetch(2 * s + 6);
@@ -584,9 +587,24 @@ int bnh_wino_f16(const uint16_t *x, long long x_ws, int H, int W, int ldx, const
                     P->K % 4 == 0 && ldo % 4 == 0 && ((uintptr_t)out & 7) == 0 && (B == 1 || o_ws % 4 == 0) &&
                     (!res || (ldr % 4 == 0 && ((uintptr_t)res & 7) == 0 && (B == 1 || r_ws % 4 == 0)));
   if (r_ok && !v1) {
+    // Few strips leave CUs idle while each block walks its whole image (9 windows of 96 x 128 px, 36 strips: 84 us),
+    // so a strip's tile rows are split over nseg blocks. A block's cost is its rows + 2.5 (its U fragments and first
+    // four input rows); blocks that share a CU each run slower: per block, k on a CU cost 0.85 k of one alone (0.55 k
+    // with at most 32 input channels, whose blocks are small). The split with the least cost on the fullest CU: that
+    // launch 20.7 us in 7 (22.4 in 6, 25.0 in 8), one window 82 -> 9.8 us in 24, 20 windows 84.5 -> 30 us in 3, and no
+    // split from about 256 strips on (64 windows of 96 x 256 px: 122 us, 127 us in 2). Rows do not depend on the split.
+    const long long cols = (long long)strips * B;
+    int nseg = 1;
+    double least = 0;
+    for (int n = 1; n <= (H / 2 + 1) / 2 && (n == 1 || cols * n <= 2048); n++) {
+      const double cu = (double)bnh_ceil_div(cols * n, 256), share = nch == 1 ? 0.55 : 0.85;
+      const double cost = (bnh_ceil_div(H / 2, n) + 2.5) * (cu > 1 ? share * cu : 1.0);
+      if (n == 1 || cost < least) least = cost, nseg = n;
+    }
+    const dim3 rgrid((unsigned)(cols * nseg));
 #define WINOR_A(NCH, NCB, ACT)                                                                                         \
-  hipLaunchKernelGGL((k_wino_f16r<NCH, NCB, ACT>), grid, dim3(256), 0, st, x, x_ws, H, W, P->C, ldx, P->U, P->b, P->K, \
-                     out, o_ws, ldo, opad, res, r_ws, ldr, rpad, strips)
+  hipLaunchKernelGGL((k_wino_f16r<NCH, NCB, ACT>), rgrid, dim3(256), 0, st, x, x_ws, H, W, P->C, ldx, P->U, P->b,      \
+                     P->K, out, o_ws, ldo, opad, res, r_ws, ldr, rpad, strips, nseg)
 #define WINOR(NCH, NCB)                                                                                                \
   do {                                                                                                                 \
     if (act == 1) WINOR_A(NCH, NCB, 1);                                                                                \

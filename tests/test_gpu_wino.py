@@ -102,6 +102,29 @@ def test_within_stated_tolerance(hip, H, W, C, K):
         assert (err <= tol).all(), float(np.max(err / tol))
 
 
+@pytest.mark.parametrize("H,W,C,K,rpad", [(2, 70, 64, 64, 0), (6, 34, 24, 24, 1), (46, 34, 64, 64, 0),
+                                          (94, 30, 32, 48, 1)])
+def test_row_segments(hip, H, W, C, K, rpad):
+    """Few strips: each strip's tile rows are split over blocks (segments of two rows and more, uneven ones). The
+    rows do not depend on the split: one window and three equal the same windows of a batch long enough (260 strips
+    and more) to run unsplit, byte for byte, with a residual, SiLU and a zero halo"""
+    rng = np.random.default_rng(H + W)
+    n = 260 // ((W // 2 + 15) // 16) + 1
+    xp, w, b = make(rng, 3, H, W, C, K)
+    res = np.zeros((3, H + 2 * rpad, W + 2 * rpad, K), np.float16)
+    res[:] = rng.standard_normal(res.shape)
+    idx = np.arange(n) % 3
+    say("wino segments", H, W, C, K, n)
+    whole = run(hip, xp[idx], w, b, act=1, opad=1, res=res[idx], rpad=rpad)
+    three = run(hip, xp, w, b, act=1, opad=1, res=res, rpad=rpad)
+    one = run(hip, xp[2:], w, b, act=1, opad=1, res=res[2:], rpad=rpad)
+    assert np.array_equal(three.view(np.uint16), whole[:3].view(np.uint16))
+    assert np.array_equal(one.view(np.uint16), whole[2:3].view(np.uint16))
+    plain = run(hip, xp, w, b).astype(np.float64)
+    ref = np.stack([direct(xp[i].astype(np.float64), w, b).reshape(H, W, K) for i in range(3)])
+    assert np.abs(plain - ref).max() <= 8 * 2.0 ** -11 * np.abs(ref).max()   # the whole-output bound used below
+
+
 def test_epilogue_forms(hip):
     rng = np.random.default_rng(3)
     B, H, W, C, K = 2, 6, 8, 16, 32
