@@ -10,6 +10,8 @@
 // the reference's order; a thread per (window, channel) re-reads the outputs and adds them up that way.
 #include <string.h>
 
+#include <type_traits>
+
 #include "bnh_internal.h"
 #include "bnh_num.h"
 
@@ -730,246 +732,183 @@ __global__ __launch_bounds__(256) void k_dw_f16v(const h16 *__restrict__ xp, lon
 //   form 2 (fp32 DW3): every pixel in raster order;
 //   form 1 (fp16 DWK): per row fp16 group sums (o0 + o1) + (o2 + o3), then an fp16 pair, then a single, widened;
 //   form 3 (fp16 DW3): per row an fp16 running sum over the row, widened at the row's end.
-// The sum is one dependent chain per channel. A block owns one window and a slab of <= 64 channels: all its waves
-// compute the terms of a chunk of rows into LDS (4 channels per item, vector loads), then wave 0 (one lane per
-// channel) adds them in order while the other waves compute the next chunk into the second buffer.
+// The sum is one dependent chain per channel, so a launch is bound by its chains' adds (few windows) or by reading
+// the outputs once (many). A block owns S channels of one window: its waves turn outputs into terms and lay them in
+// LDS channel by channel, and wave 0, a lane per channel, adds them in order, four terms a 16-byte LDS read, the next
+// 16 terms' reads behind the adds of the last 16. Images of several chunks run pipelined: while wave 0 adds chunk i,
+// waves 1..3 write chunk i + 1 into the other buffer and keep the loads of chunk i + 2 in flight in registers across
+// the barrier. A dependent add takes 2.84 ns here, 45 us for 249 x 63 pixels in raster order.
+// Measured against one term a read with a row's bookkeeping between rows: 249 x 63 px x 40 channels (raster order)
+// 217 -> 62 us for one window, 183 -> 82 us for 128; 125 x 32 x 144 43 -> 18 and 80 -> 57; 63 x 16 x 288 (groups)
+// 20 -> 4 and 25 -> 22; fp16 64 x 24 x 288 (row sums) 29 -> 4 and 35 -> 19.
 template <int FORM>
-__device__ __forceinline__ int cs_terms(int Wo) {
+__host__ __device__ __forceinline__ int cs_terms(int Wo) {  // terms per row
   if (FORM == 0) return Wo / 4 + Wo % 4;
   if (FORM == 2) return Wo;
   if (FORM == 1) return Wo / 4 + ((Wo % 4) >> 1) + (Wo & 1);
   return 1;
 }
 
-struct f4 { float v[4]; };
+template <typename T>
+struct CsQuad;  // four channels of a pixel as loaded
+template <>
+struct CsQuad<float> {
+  float4 q;
+  BNH_DEV void load(const float *p) { q = *(const float4 *)p; }
+  BNH_DEV float at(int i) const { return i == 0 ? q.x : i == 1 ? q.y : i == 2 ? q.z : q.w; }
+};
+template <>
+struct CsQuad<h16> {
+  uint2 q;
+  BNH_DEV void load(const h16 *p) { q = *(const uint2 *)p; }
+  BNH_DEV h16 at(int i) const { return hfrom((uint16_t)((i < 2 ? q.x : q.y) >> (16 * (i & 1)))); }
+};
 
-BNH_DEV f4 cs_ld(const float *p) {
-  const float4 t = *(const float4 *)p;
-  return f4{{t.x, t.y, t.z, t.w}};
-}
-BNH_DEV void cs_ld(const h16 *p, h16 (&o)[4]) {
-  const uint2 t = *(const uint2 *)p;
-  o[0] = hfrom((uint16_t)(t.x & 0xffffu)); o[1] = hfrom((uint16_t)(t.x >> 16));
-  o[2] = hfrom((uint16_t)(t.y & 0xffffu)); o[3] = hfrom((uint16_t)(t.y >> 16));
-}
+// chunk capacity: U terms of 4 channels a loading thread holds in registers, 192 loading threads
+template <int FORM, int S>
+struct CsPlan {
+  static constexpr int U = FORM == 2 ? 8 : 4, TT = U * 192 * 4 / S;
+};
 
-// term j of a row (row points at the row's first pixel, channel c0 of the 4) for 4 channels
-template <int FORM>
-BNH_DEV f4 cs_term(const float *row, int C, int Wo, int j) {
-  const int g4 = Wo / 4;
-  if (FORM == 0 && j < g4) {
-    const f4 a = cs_ld(row + (long long)(4 * j) * C), b = cs_ld(row + (long long)(4 * j + 1) * C);
-    const f4 c = cs_ld(row + (long long)(4 * j + 2) * C), d = cs_ld(row + (long long)(4 * j + 3) * C);
-    f4 r;
-#pragma unroll
-    for (int q = 0; q < 4; q++) r.v[q] = (a.v[q] + b.v[q]) + (c.v[q] + d.v[q]);
-    return r;
-  }
-  const int ox = FORM == 0 ? 4 * g4 + (j - g4) : j;
-  return cs_ld(row + (long long)ox * C);
-}
-template <int FORM>
-BNH_DEV f4 cs_term(const h16 *row, int C, int Wo, int j) {
-  f4 r;
-  h16 a[4], b[4], c[4], d[4];
-  if (FORM == 3) {
-    h16 rs[4] = {(h16)0.0f, (h16)0.0f, (h16)0.0f, (h16)0.0f};
-    for (int ox = 0; ox < Wo; ox++) {
-      cs_ld(row + (long long)ox * C, a);
-#pragma unroll
-      for (int q = 0; q < 4; q++) rs[q] = rs[q] + a[q];
-    }
-#pragma unroll
-    for (int q = 0; q < 4; q++) r.v[q] = (float)rs[q];
-    return r;
-  }
-  const int g4 = Wo / 4, np = (Wo % 4) >> 1;
-  if (j < g4) {
-    cs_ld(row + (long long)(4 * j) * C, a);
-    cs_ld(row + (long long)(4 * j + 1) * C, b);
-    cs_ld(row + (long long)(4 * j + 2) * C, c);
-    cs_ld(row + (long long)(4 * j + 3) * C, d);
-#pragma unroll
-    for (int q = 0; q < 4; q++) r.v[q] = (float)((a[q] + b[q]) + (c[q] + d[q]));
-  } else if (j < g4 + np) {
-    cs_ld(row + (long long)(4 * g4) * C, a);
-    cs_ld(row + (long long)(4 * g4 + 1) * C, b);
-#pragma unroll
-    for (int q = 0; q < 4; q++) r.v[q] = (float)(a[q] + b[q]);
-  } else {
-    cs_ld(row + (long long)(Wo - 1) * C, a);
-#pragma unroll
-    for (int q = 0; q < 4; q++) r.v[q] = (float)a[q];
-  }
-  return r;
-}
-
-template <typename T, int FORM>
-__global__ __launch_bounds__(256) void k_chsum(const T *__restrict__ out, long long o_ws, int C, int Ho, int Wo, int R,
-                                               float *__restrict__ chsum, long long cs_ws) {
-  extern __shared__ float tb[];
+template <typename T, int FORM, int S>
+__global__ __launch_bounds__(256) void k_chsum(const T *__restrict__ out, long long o_ws, int C, int Wo, int NT, int TT,
+                                               int slabs, double rTn, float *__restrict__ chsum, long long cs_ws) {
+  extern __shared__ __attribute__((aligned(16))) float tb[];  // [1 or 2][S][TT + 4], 16 floats read past the end
+  constexpr int U = CsPlan<FORM, S>::U, NP = FORM == 2 ? 1 : 4, S4 = S / 4;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int c0 = blockIdx.x * 64, S = C - c0 < 64 ? C - c0 : 64, S4 = S / 4, win = blockIdx.y;
-  const int Tn = cs_terms<FORM>(Wo), per = R * Tn * S, nch = (Ho + R - 1) / R;
+  const unsigned lb = bnh_xcd_block(blockIdx.x, gridDim.x);  // a window's slabs share pixels' cache lines: one XCD
+  const int win = (int)(lb / slabs), c0 = (int)(lb % slabs) * S, ST = TT + 4, per = S * ST;
+  const int items = TT * S4, nch = (NT + TT - 1) / TT;
   const T *o = out + win * o_ws + c0;
-  // a chunk's terms: each thread takes items t0, t0 + nt, ...; CB items' loads are issued before any of their LDS
-  // stores, so that a thread keeps CB loads (4 CB for the 4-pixel terms) in flight
-  constexpr int CB = FORM == 2 ? 16 : 4;
-  auto load = [&](int ch, int t0, int nt) {
-    const int rows = Ho - ch * R < R ? Ho - ch * R : R;
-    float *buf = tb + (ch & 1) * per;
-    const int n = rows * Tn * S4;
-    for (int base = t0; base < n; base += CB * nt) {
-      f4 v[CB];
+  const int Tn = cs_terms<FORM>(Wo), g4 = Wo / 4, np = (Wo % 4) >> 1;
+  const bool whole = Wo % 4 == 0;  // rows of whole groups: group t is pixels 4 t .. 4 t + 3 of the image
+  CsQuad<T> v[U][NP];
+  int kind[U];  // 4, 2 or 1 pixels in the term
+  auto fetch = [&](int ch, int l, int nl) {
 #pragma unroll
-      for (int u = 0; u < CB; u++) {
-        const int it = base + u * nt;
-        if (it < n) {
-          const int c4 = it % S4, j = (it / S4) % Tn, r = it / (S4 * Tn);
-          v[u] = cs_term<FORM>(o + (long long)(ch * R + r) * Wo * C + 4 * c4, C, Wo, j);
-        }
+    for (int u = 0; u < U; u++) {
+      const int it = l + u * nl;
+      if (it >= items) break;
+      const int cq = it % S4, t_ = ch * TT + it / S4, t = t_ < NT ? t_ : NT - 1;  // terms past NT are not added
+      const T *p = o + (c0 + 4 * cq < C ? 4 * cq : 0);
+      if (FORM == 2) {
+        v[u][0].load(p + (long long)t * C);
+        continue;
       }
+      int px = 4 * t, k = 4;
+      if (!whole) {
+        const int y = bnh_div(t, Tn, rTn), j = t - y * Tn;
+        px = y * Wo + (j < g4 ? 4 * j : FORM == 0 ? 3 * g4 + j : j < g4 + np ? 4 * g4 : Wo - 1);
+        k = j < g4 ? 4 : FORM == 1 && j < g4 + np ? 2 : 1;
+      }
+      kind[u] = k;
 #pragma unroll
-      for (int u = 0; u < CB; u++) {
-        const int it = base + u * nt;
-        if (it < n) {
-          const int c4 = it % S4, j = (it / S4) % Tn, r = it / (S4 * Tn);
-          *(float4 *)(buf + (r * Tn + j) * S + 4 * c4) = make_float4(v[u].v[0], v[u].v[1], v[u].v[2], v[u].v[3]);
+      for (int i = 0; i < NP; i++) v[u][i].load(p + (long long)(px + (i < k ? i : 0)) * C);
+    }
+  };
+  auto write = [&](float *buf, int l, int nl) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int it = l + u * nl;
+      if (it >= items) break;
+      float *d = buf + 4 * (it % S4) * ST + it / S4;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const T a = v[u][0].at(q);
+        float f;
+        if (FORM == 2) f = (float)a;
+        else {
+          const T b = v[u][1 % NP].at(q), c = v[u][2 % NP].at(q), e = v[u][3 % NP].at(q);
+          f = (float)((a + b) + (c + e));
+          if (!whole) f = kind[u] == 4 ? f : FORM == 1 && kind[u] == 2 ? (float)(a + b) : (float)a;
         }
+        d[q * ST] = f;
       }
     }
   };
-  load(0, tid, 256);
-  __syncthreads();
+  // form 3's terms: a row's fp16 running sum, 8 pixels' loads in flight
+  auto rows = [&](int ch, float *buf, int l, int nl) {
+    for (int it = l; it < items; it += nl) {
+      const int cq = it % S4, t = ch * TT + it / S4;
+      if (t >= NT) break;
+      const T *p = o + (c0 + 4 * cq < C ? 4 * cq : 0) + (long long)t * Wo * C;
+      T rs[4] = {(T)0.0f, (T)0.0f, (T)0.0f, (T)0.0f};
+      for (int x = 0; x < Wo; x += 8) {
+        CsQuad<T> a[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) a[i].load(p + (long long)(x + i < Wo ? x + i : Wo - 1) * C);
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+          if (x + i < Wo) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) rs[q] = rs[q] + a[i].at(q);
+          }
+      }
+      float *d = buf + 4 * cq * ST + it / S4;
+#pragma unroll
+      for (int q = 0; q < 4; q++) d[q * ST] = (float)rs[q];
+    }
+  };
+  // LDS only: a load in flight into registers stays in flight across the barrier
+  auto barrier = [] {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  const int l = tid - 64;  // a loading thread's index once wave 0 adds
+  if (FORM == 3) rows(0, tb, tid, 256);
+  else {
+    fetch(0, tid, 256);
+    write(tb, tid, 256);
+    if (nch > 1 && wave) fetch(1, l, 192);
+  }
+  if (nch > 1 && !wave) __builtin_amdgcn_s_setprio(3);
+  barrier();
   float cs = 0.f;
   for (int ch = 0; ch < nch; ch++) {
-    if (wave != 0) {
-      if (ch + 1 < nch) load(ch + 1, tid - 64, 192);
-    } else if (lane < S) {
-      const int rows = Ho - ch * R < R ? Ho - ch * R : R;
-      const float *buf = tb + (ch & 1) * per + lane;
-      const int n = rows * Tn;
-      int it = 0;
-      for (; it + 16 <= n; it += 16) {  // sixteen LDS reads in flight, then the sixteen dependent adds in order
-        float t[16];
-#pragma unroll
-        for (int u = 0; u < 16; u++) t[u] = buf[(it + u) * S];
-#pragma unroll
-        for (int u = 0; u < 16; u++) cs = cs + t[u];
-      }
-      for (; it < n; it++) cs = cs + buf[it * S];
-    }
-    __syncthreads();
-  }
-  if (wave == 0 && lane < S) chsum[win * cs_ws + c0 + lane] = cs;
-}
-
-// fp32 channel sums, wave-private form (FORM 0 / 2, Wo <= 64): a wave owns 16 channels of one window and walks its
-// image rows in order. Lane l loads the 16 channels' float4 quad (l & 3) of pixels 16 i + (l >> 2); 8 rows of those
-// loads stay in flight in a register ring, so the wave keeps 8 x Wo x 64 bytes on the way (no LDS double buffer
-// bounds it). A row that has landed goes through a wave-private LDS row [Wo][16], from which lanes 0..15 (one per
-// channel) add the row's terms to their running sums in the reference's order: DW3 every pixel, DWK each 4-pixel
-// group as (o0 + o1) + (o2 + o3), then the tail pixels. No block barrier: a wave's LDS writes and reads are in order.
-template <int FORM, int NI>
-__global__ __launch_bounds__(256) void k_chsum_w(const float *__restrict__ out, long long o_ws, int C, int Ho, int Wo,
-                                                 float *__restrict__ chsum, long long cs_ws) {
-  constexpr int NR = 8;  // rows in flight (the ring's loop is unrolled: longer rings land in scratch memory)
-  __shared__ float rowb[4][64 * 16];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, win = blockIdx.y;
-  const int c0 = blockIdx.x * 64 + wave * 16;
-  if (c0 >= C) return;
-  const int nc = C - c0 < 16 ? C - c0 : 16;  // a multiple of 4
-  const int p16 = lane >> 2, cq = lane & 3;
-  // every lane loads (no branch, so the loads' counters stay exact and the ring stays in flight): rows past the image,
-  // pixels past the row and quads past the channels read a valid address whose value no sum uses
-  const float *img = out + win * o_ws + c0;  // wave-uniform
-  int lofs[NI];                              // per lane: pixel 16 i + (l >> 2), quad (l & 3), in floats
-#pragma unroll
-  for (int i = 0; i < NI; i++) {
-    const int px = 16 * i + p16;
-    lofs[i] = (px < Wo ? px : Wo - 1) * C + 4 * (4 * cq < nc ? cq : 0);
-  }
-  float *rb = rowb[wave];
-  float4 v[NR][NI];
-  auto rowp = [&](int y) { return img + (long long)(y < Ho ? y : Ho - 1) * Wo * C; };  // wave-uniform
-#pragma unroll
-  for (int s = 0; s < NR; s++) {
-    const float *rp = rowp(s);
-#pragma unroll
-    for (int i = 0; i < NI; i++)  // (the select keeps the compiler from placing the ring in scratch memory)
-      v[s][i] = s < Ho ? *(const float4 *)(rp + lofs[i]) : make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-  const int g4 = Wo & ~3;
-  float cs = 0.f;
-  for (int y0 = 0; y0 < Ho; y0 += NR) {
-#pragma unroll
-    for (int s = 0; s < NR; s++) {
-      const int y = y0 + s;
-      if (y >= Ho) break;
-#pragma unroll
-      for (int i = 0; i < NI; i++) *(float4 *)(rb + (16 * i + p16) * 16 + 4 * cq) = v[s][i];  // px < 64: in the row
-      {  // the ring slot's next row
-        const float *rp = rowp(y + NR);
-#pragma unroll
-        for (int i = 0; i < NI; i++) v[s][i] = *(const float4 *)(rp + lofs[i]);
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      if (NI < 4 && lane < nc) {  // rows of at most 32 pixels: 16 LDS reads in flight, then their adds in order
-        const float *col = rb + lane;
-        if (FORM == 2) {
-          int x = 0;
-          for (; x + 16 <= Wo; x += 16) {
-            float t[16];
-#pragma unroll
-            for (int u = 0; u < 16; u++) t[u] = col[(x + u) * 16];
-#pragma unroll
-            for (int u = 0; u < 16; u++) cs = cs + t[u];
-          }
-          for (; x < Wo; x++) cs = cs + col[x * 16];
-        } else {
-          for (int x = 0; x < g4; x += 4) {
-            const float a = col[x * 16], b = col[(x + 1) * 16], c2 = col[(x + 2) * 16], d = col[(x + 3) * 16];
-            cs = cs + ((a + b) + (c2 + d));
-          }
-          for (int x = g4; x < Wo; x++) cs = cs + col[x * 16];
+    if (wave) {
+      if (ch + 1 < nch) {
+        float *buf = tb + ((ch + 1) & 1) * per;
+        if (FORM == 3) rows(ch + 1, buf, l, 192);
+        else {
+          write(buf, l, 192);
+          if (ch + 2 < nch) fetch(ch + 2, l, 192);
         }
       }
-      if (NI == 4 && lane < nc) {
-        // rows of up to 64 pixels (the widest images, fewest waves): all the row's terms read from LDS at once (one
-        // LDS round trip per row; 238 -> 193 us for 40 channels of 249 x 63 pixels), then added in order; reads past
-        // the row's Wo pixels stay inside the wave's LDS row and are not used
-        const float *col = rb + lane;
-        float t[16 * NI];
+    } else {
+      const float *row = tb + (ch & 1) * per + (lane % S) * ST;
+      const int n = NT - ch * TT < TT ? NT - ch * TT : TT;
+      const float4 *p = (const float4 *)row;
+      float4 a[4], b[4];
+      auto read = [&](float4 (&d)[4], int t4) {
 #pragma unroll
-        for (int u = 0; u < 16 * NI; u++) t[u] = col[u * 16];
-        if (FORM == 2) {
+        for (int i = 0; i < 4; i++) d[i] = p[t4 + i];
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto add = [&](const float4 (&d)[4]) {
 #pragma unroll
-          for (int u = 0; u < 16 * NI; u++)
-            if (u < Wo) cs = cs + t[u];
-        } else {
-#pragma unroll
-          for (int u = 0; u < 16 * NI; u += 4)
-            if (u + 4 <= g4) cs = cs + ((t[u] + t[u + 1]) + (t[u + 2] + t[u + 3]));
-#pragma unroll
-          for (int u = 0; u < 16 * NI; u++)
-            if (u >= g4 && u < Wo) cs = cs + t[u];
+        for (int i = 0; i < 4; i++) {
+          cs = cs + d[i].x;
+          cs = cs + d[i].y;
+          cs = cs + d[i].z;
+          cs = cs + d[i].w;
         }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      int t = 0;
+      read(a, 0);
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): only the loop's own reads pend in it, so its waits count them
+      for (; t + 32 <= n; t += 32) {  // 16 terms' reads in flight behind the adds of the 16 before them
+        read(b, t / 4 + 4);
+        add(a);
+        read(a, t / 4 + 8);
+        add(b);
       }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      for (; t < n; t++) cs = cs + row[t];
     }
+    if (ch + 1 < nch) barrier();
   }
-  if (lane < nc) chsum[win * cs_ws + c0 + lane] = cs;
-}
-
-// rows per chunk: two buffers of at most `cap` floats
-static int chsum_rows(int Tn, int S, int Ho, int cap) {
-  int R = cap / (Tn * S);
-  if (R < 1) R = 1;
-  return R < Ho ? R : Ho;
+  if (!wave && lane < S && c0 + lane < C) chsum[win * cs_ws + c0 + lane] = cs;
 }
 
 // one thread per (window, channel) walking the whole image: for channel counts that are not a multiple of 4
@@ -1022,9 +961,7 @@ __global__ void k_chsum1_f16(const h16 *__restrict__ out, long long o_ws, int C,
 template <typename T, int FORM>
 static int chsum_launch(const T *out, long long o_ws, int C, int Ho, int Wo, float *chsum, long long cs_ws, int B,
                         hipStream_t st) {
-  const int Tn = FORM == 0 ? Wo / 4 + Wo % 4 : FORM == 2 ? Wo : FORM == 1 ? Wo / 4 + ((Wo % 4) >> 1) + (Wo & 1) : 1;
-  const int S = C < 64 ? C : 64;
-  if (C % 4 || ((uintptr_t)out & (4 * sizeof(T) - 1)) || (B > 1 && o_ws % 4) || Tn * S > 8192) {
+  if (C % 4 || ((uintptr_t)out & (4 * sizeof(T) - 1)) || (B > 1 && o_ws % 4)) {
     if (sizeof(T) == 4)
       hipLaunchKernelGGL(k_chsum1_f32, dim3((unsigned)bnh_ceil_div((long long)B * C, 256)), dim3(256), 0, st,
                          (const float *)out, o_ws, C, Ho, Wo, FORM, chsum, cs_ws, B);
@@ -1034,29 +971,21 @@ static int chsum_launch(const T *out, long long o_ws, int C, int Ho, int Wo, flo
     BNH_HIP(hipGetLastError());
     return 0;
   }
-  // fp32 sums over rows of at most 64 pixels: the wave-private form, from 33 channels up (with fewer, two waves per
-  // window keep too little in flight: 24 channels of 249 x 63 pixels take about 177 us there against 166 us below)
-  if constexpr (sizeof(T) == 4 && (FORM == 0 || FORM == 2)) {
-    if (Wo <= 64 && C > 32) {
-      const dim3 grid((unsigned)bnh_ceil_div(C, 64), (unsigned)B);
-      const float *o = (const float *)out;
-      if (Wo <= 16) hipLaunchKernelGGL((k_chsum_w<FORM, 1>), grid, dim3(256), 0, st, o, o_ws, C, Ho, Wo, chsum, cs_ws);
-      else if (Wo <= 32) hipLaunchKernelGGL((k_chsum_w<FORM, 2>), grid, dim3(256), 0, st, o, o_ws, C, Ho, Wo, chsum, cs_ws);
-      else hipLaunchKernelGGL((k_chsum_w<FORM, 4>), grid, dim3(256), 0, st, o, o_ws, C, Ho, Wo, chsum, cs_ws);
-      BNH_HIP(hipGetLastError());
-      return 0;
-    }
-  }
-  // a block's chunk is one memory round trip of its loading waves: with at most one block per CU (no more blocks
-  // than 2 per CU in the launch) the chunks take up to 144 KB of LDS, else 64 KB so that several blocks share a CU
-  const long long nblk = bnh_ceil_div(C, 64) * (long long)B;
-  const int cap = nblk <= 512 ? 18432 : 8192;
-  const int R = chsum_rows(Tn, S, Ho, cap);
-  const size_t lds = 2 * sizeof(float) * (size_t)R * Tn * S;
-  if (lds > 64 * 1024)
-    BNH_HIP(hipFuncSetAttribute((const void *)k_chsum<T, FORM>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL((k_chsum<T, FORM>), dim3((unsigned)bnh_ceil_div(C, 64), (unsigned)B), dim3(256), lds, st, out,
-                     o_ws, C, Ho, Wo, R, chsum, cs_ws);
+  const int Tn = cs_terms<FORM>(Wo), NT = Ho * Tn;
+  auto launch = [&](auto s_) {
+    constexpr int S = decltype(s_)::value, most = CsPlan<FORM, S>::TT;
+    const int TT = NT < most ? (int)bnh_round_up(NT, 4) : most, slabs = (int)bnh_ceil_div(C, S);
+    const size_t lds = 4 * ((size_t)(NT > TT ? 2 : 1) * S * (TT + 4) + 16);
+    hipLaunchKernelGGL((k_chsum<T, FORM, S>), dim3((unsigned)((long long)slabs * B)), dim3(256), lds, st, out, o_ws, C,
+                       Wo, NT, TT, slabs, 1.0 / Tn, chsum, cs_ws);
+  };
+  // More channels a block load longer runs of a pixel, fewer make more blocks and longer chunks (a chunk costs its
+  // barrier). 64 from four blocks a CU on for images of one chunk (128 windows of 16 x 4 x 1392: 9.8 us, 12.7 with 32,
+  // 20.5 with 16), 32 from two a CU on (128 of 125 x 32 x 192: 75 us, 77 with 64, 88 with 16), else 16 (128 of
+  // 249 x 63 x 40: 82 us, 92 with 32; one window of it: 63 us, 71 with 32, 166 with 64).
+  if (bnh_ceil_div(C, 64) * B >= 1024 && NT <= CsPlan<FORM, 64>::TT) launch(std::integral_constant<int, 64>{});
+  else if (bnh_ceil_div(C, 32) * B >= 512) launch(std::integral_constant<int, 32>{});
+  else launch(std::integral_constant<int, 16>{});
   BNH_HIP(hipGetLastError());
   return 0;
 }

@@ -157,6 +157,27 @@ def test_dw3(hip, dtype, s):
         check_case(hip, "dw3", dtype, 2, H, W, C, 3, s, pt, pl, 1, seed=H + W + s)
 
 
+@pytest.mark.parametrize("form,dtype,B,H,W,C,k", [
+    ("dw3", np.float32, 2, 6, 64, 20, 3),      # 16-channel blocks (the last one of 4): 384 terms, one whole chunk
+    ("dw3", np.float32, 2, 5, 77, 20, 3),      # 385: one term in the second chunk
+    ("dw3", np.float32, 2, 31, 50, 16, 3),     # 1550: five chunks
+    ("dw3", np.float32, 512, 8, 24, 12, 3),    # 32-channel blocks: 192 terms, one whole chunk
+    ("dw3", np.float32, 512, 13, 16, 36, 3),   # 208, and a second block of 4 channels
+    ("dw3", np.float32, 1024, 12, 8, 8, 3),    # 64-channel blocks: 96 terms, one whole chunk
+    ("dwk", np.float32, 2, 24, 32, 24, 5),     # groups of 4: 192 terms, one whole chunk of a 16-channel block
+    ("dwk", np.float32, 2, 13, 61, 24, 5),     # 16 terms a row (15 groups, one tail pixel): 208
+    ("dwk", np.float32, 512, 14, 31, 8, 3),    # 10 terms a row: 140 (chunks of 96)
+    ("dwk", np.float32, 1024, 12, 16, 4, 3),   # 48 terms, one whole chunk of a 64-channel block
+    ("dwk", np.float16, 2, 13, 63, 24, 5),     # fp16 groups, a pair and a single: 17 terms a row
+    ("dwk", np.float16, 1024, 5, 7, 72, 3),
+    ("dw3", np.float16, 2, 200, 9, 24, 3),     # row sums: 200 rows, two chunks of a 16-channel block
+    ("dw3", np.float16, 512, 97, 3, 8, 3),     # 97 rows: two chunks of a 32-channel block
+    ("dw3", np.float16, 1024, 3, 17, 4, 3)])
+def test_channel_sums_chunks(hip, form, dtype, B, H, W, C, k):
+    """The channel sums at the edges of their chunks, for each block width, at both ends of the batch"""
+    check_case(hip, form, dtype, B, H, W, C, k, 1, k // 2, k // 2, 1, seed=H + W + C, windows=[0, B - 1])
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float16])
 @pytest.mark.parametrize("form", ["dwk", "dw3"])
 def test_dw_specials(hip, dtype, form):
