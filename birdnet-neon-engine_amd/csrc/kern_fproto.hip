@@ -6,17 +6,22 @@
 //
 // Bit-identical to the reference. Every product sum is one fused multiply-add chain in the reference's order: fp32
 // from +0 over k; fp16 from +0 over each K block (the fp16 GEMM's balanced blocks of at most 128 steps), the blocks'
-// widened results summed in fp32 from +0. Matrix cores sum their products in an order of their own, so the chains
-// run on the VALU: a thread owns 8 cells x 8 prototypes (64 fp32 chains, or 32 packed fp16 pairs), its operands two
-// 16-byte LDS reads per k step each. The maximum over cells is exact and order-free (NaN-propagating FMAX).
+// widened results summed in fp32 from +0. The maximum over cells is exact and order-free (NaN-propagating FMAX).
 //
-// Prototypes are repacked at load into k-major rows [K][Npt] (Npt = Np rounded up to 256, zeros past Np): a block's
-// 256 prototypes at one k are one contiguous 1 KB (fp32) or 512 B (fp16) run. A block is one window x 256
-// prototypes, windows fastest, so the blocks in flight share their prototype tile in L2; it walks the window's cells
-// 64 at a time.
+// The fp32 chains run on the matrix cores: v_mfma_f32_16x16x4_f32 adds its four products one after the other in k
+// order, each a fused multiply-add rounded to nearest even, denormals kept (compared bit for bit with fmaf chains).
+// fp16 matrix instructions accumulate in fp32, so the fp16 chains run on the VALU: a thread owns 8 cells x 8
+// prototypes (32 packed fp16 pairs), its operands two 16-byte LDS reads per k step each.
+//
+// Prototypes are repacked at load: kinds 0 and 1 into tiles of 16 prototypes x 16 k in the matrix instruction's
+// operand order (lane (c, h) of a wave reads prototype c at k = h, 4 + h, 8 + h, 12 + h as one 16- or 8-byte word,
+// zeros past Np and K); kind 2 into k-major rows [K][Npt] (Npt = Np rounded up to 256, zeros past Np), a block's 256
+// prototypes at one k one contiguous 512 B run.
 #include <math.h>
 #include <stdlib.h>
 #include <string.h>
+
+#include <type_traits>
 
 #include "bnh_f16.h"
 #include "bnh_internal.h"
@@ -26,7 +31,7 @@ struct bnh_fproto {
   int kind;     // 0 fp32 (PROTO variant 0), 1 fp16-stored / fp32 math (PROTO_F32H), 2 fp16 (PROTO variant 1)
   int Np, K, Npt;
   int nblk, bs;  // kind 2: the fp16 GEMM's K blocks
-  void *w;       // k-major [K][Npt]: fp32 (kind 0) or fp16 bit patterns (kinds 1, 2)
+  void *w;       // kinds 0, 1: [Np/16][K/16][64 lanes][4] (fp32, fp16 bit patterns); kind 2: k-major [K][Npt] fp16
 };
 
 // ------------------------------------------------------------------ L2 normalisation of the cells
@@ -69,121 +74,202 @@ __global__ __launch_bounds__(256) void k_l2norm(const void *__restrict__ xv, lon
   }
 }
 
+#define FP_BM 64   // cells per tile of the fp16 kernel
+#define FP_BN 256  // prototypes per block of the fp16 kernel
+
 // ------------------------------------------------------------------ fp32 column maxima (kinds 0 and 1)
-#define FP_BM 64   // cells per tile
-#define FP_BN 256  // prototypes per block
-#define FP_KC 16   // k steps per LDS stage
-#define FP_AS 68   // As row stride in floats ([k][cell]; 16-byte aligned rows)
-// WH: prototypes stored as fp16, widened exactly as they are staged (PROTO_F32H)
-template <bool WH>
+#define FF_KC 64           // k steps per LDS stage
+#define FF_RS (FF_KC + 4)  // LDS row stride in floats: neighbouring cells four banks apart
+typedef float fp_f4 __attribute__((ext_vector_type(4)));
+// A wave owns TC x 16 cells by TN x 16 prototypes of one window and walks the window's cells 16 TC WC at a time; the
+// block's 4 waves lie WC down the cells and 4 / WC across the prototypes. Cells go through LDS (every wave of a cell
+// group reads them), a cell's k stored by k % 4, the instruction's operand lane, so that a lane reads its four steps of
+// 16 k at once; prototypes go straight to registers; both are fetched a chunk ahead. WH: prototypes stored as fp16, widened
+// exactly (PROTO_F32H). Bound by the matrix cores' 64 fp32 multiply-adds a clock and SIMD; the vector unit's 16 and
+// an LDS read per 4 of them bounded the kernel before.
+template <bool WH, int TC, int WC, int TN>
 __global__ __launch_bounds__(256) void k_colmax_f32(const float *__restrict__ a, long long a_ws, int P, int K,
-                                                    const void *__restrict__ wv, int Npt, int Np,
-                                                    float *__restrict__ colmax, long long cm_ws, int B) {
-  __shared__ __attribute__((aligned(16))) float As[2][FP_KC][FP_AS];
-  __shared__ __attribute__((aligned(16))) float Ws[2][FP_KC][FP_BN];
-  const int tid = threadIdx.x, cg = tid & 7, pg = tid >> 3;
-  const int win = (int)(blockIdx.x % (unsigned)B), n0 = (int)(blockIdx.x / (unsigned)B) * FP_BN;
+                                                    const void *__restrict__ wv, int Np, float *__restrict__ colmax,
+                                                    long long cm_ws, int B) {
+  constexpr int WN = 4 / WC, BM = 16 * TC * WC, NL = BM / 16;
+  __shared__ __attribute__((aligned(16))) float As[2][BM * FF_RS];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c16 = lane & 15, h = lane >> 4;
+  const int wc = wave / WN, wn = wave % WN;
+  // windows fastest, and neighbouring blocks under one L2: they read the same prototypes
+  const unsigned blk = bnh_xcd_block(blockIdx.x, gridDim.x);
+  const int win = (int)(blk % (unsigned)B);
+  const int t0 = ((int)(blk / (unsigned)B) * WN + wn) * TN;  // this wave's first prototype tile
+  const int K16 = (K + 15) / 16, ntile = (Np + 15) / 16;
   const float *aw = a + win * a_ws;
-  // loader roles: A, cell tid / 4 and k 4 (tid % 4) .. + 3; W fp32, rows (tid + 256 j) / 64, 4 prototypes each;
-  // W fp16, rows (tid + 256 j) / 32, 8 prototypes each
-  const int la_c = tid >> 2, la_k = 4 * (tid & 3);
-  float4 ra;
-  float4 rw[WH ? 1 : 4];
-  uint4 rh[WH ? 2 : 1];
-  float mx[8];
+  // loader: 4 k of a cell each, 16 cells x 16 k a wave (their LDS writes fall into 64 banks)
+  auto cell_of = [&](int j) { return (tid + 256 * j) % (4 * BM) >> 2; };
+  auto quad_of = [&](int j) { return (tid + 256 * j) / (4 * BM) * 4 + (tid & 3); };
+  size_t wt[TN];  // tiles past the last repeat it, unused
 #pragma unroll
-  for (int j = 0; j < 8; j++) mx[j] = -INFINITY;
-  for (int m0 = 0; m0 < P; m0 += FP_BM) {
-    const int crow = m0 + la_c < P ? m0 + la_c : P - 1;  // rows past P repeat the last cell; their sums are unused
-    const float *arow = aw + (long long)crow * K;
-    auto load = [&](int k0) {
-      ra = k0 + la_k < K ? *(const float4 *)(arow + k0 + la_k) : make_float4(0.f, 0.f, 0.f, 0.f);
-      if (WH) {
+  for (int t = 0; t < TN; t++) wt[t] = (size_t)(t0 + t < ntile ? t0 + t : ntile - 1) * K16 * 64 + lane;
+  float4 ra[NL];
+  // this wave's prototypes of an even and an odd chunk: each 16 k reloaded for two chunks on as soon as they are used
+  using wq = std::conditional_t<WH, uint2, float4>;
+  wq w[2][TN][4];
+  float mx[TN];
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-          const int i = tid + 256 * j, row = i >> 5, c8 = i & 31;
-          rh[j] = k0 + row < K ? *(const uint4 *)((const uint16_t *)wv + (long long)(k0 + row) * Npt + n0 + 8 * c8)
-                               : make_uint4(0, 0, 0, 0);
-        }
-      } else {
+  for (int t = 0; t < TN; t++) mx[t] = -INFINITY;
+  for (int m0 = 0; m0 < P; m0 += BM) {
+    auto fetch_a = [&](int k0) {  // rows past P repeat the last cell; k past K: in bounds, unused
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const int i = tid + 256 * j, row = i >> 6, c4 = i & 63;
-          rw[j] = k0 + row < K ? *(const float4 *)((const float *)wv + (long long)(k0 + row) * Npt + n0 + 4 * c4)
-                               : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
+      for (int j = 0; j < NL; j++) {
+        const int k = k0 + 4 * quad_of(j) < K ? k0 + 4 * quad_of(j) : K - 4;
+        const int r = m0 + cell_of(j) < P ? m0 + cell_of(j) : P - 1;
+        ra[j] = *(const float4 *)(aw + (long long)r * K + k);
       }
     };
-    auto store = [&](int buf) {
-      As[buf][la_k + 0][la_c] = ra.x;
-      As[buf][la_k + 1][la_c] = ra.y;
-      As[buf][la_k + 2][la_c] = ra.z;
-      As[buf][la_k + 3][la_c] = ra.w;
-      if (WH) {
+    auto commit_a = [&](int buf) {
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-          const int i = tid + 256 * j, row = i >> 5, c8 = i & 31;
-          const h2 v[4] = {__builtin_bit_cast(h2, rh[j].x), __builtin_bit_cast(h2, rh[j].y),
-                           __builtin_bit_cast(h2, rh[j].z), __builtin_bit_cast(h2, rh[j].w)};
-          *(float4 *)&Ws[buf][row][8 * c8] = make_float4((float)v[0].x, (float)v[0].y, (float)v[1].x, (float)v[1].y);
-          *(float4 *)&Ws[buf][row][8 * c8 + 4] = make_float4((float)v[2].x, (float)v[2].y, (float)v[3].x, (float)v[3].y);
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const int i = tid + 256 * j, row = i >> 6, c4 = i & 63;
-          *(float4 *)&Ws[buf][row][4 * c4] = rw[j];
-        }
+      for (int j = 0; j < NL; j++) {
+        float *d = &As[buf][cell_of(j) * FF_RS + quad_of(j)];
+        d[0] = ra[j].x, d[16] = ra[j].y, d[32] = ra[j].z, d[48] = ra[j].w;
       }
     };
-    float acc[8][8];
+    auto fetch_w = [&](int set, int g, int k0) {
+      const int kt = k0 / 16 + g < K16 ? k0 / 16 + g : K16 - 1;
 #pragma unroll
-    for (int i = 0; i < 8; i++)
+      for (int t = 0; t < TN; t++) w[set][t][g] = ((const wq *)wv)[wt[t] + (size_t)kt * 64];
+    };
+    fp_f4 acc[TC][TN];
 #pragma unroll
-      for (int j = 0; j < 8; j++) acc[i][j] = 0.f;
-    __syncthreads();  // the previous tile's last reads of buffer 0 are done
-    load(0);
-    store(0);
+    for (int i = 0; i < TC; i++)
+#pragma unroll
+      for (int t = 0; t < TN; t++) acc[i][t] = (fp_f4){0.f, 0.f, 0.f, 0.f};
+    // the chunk at k0 in LDS buffer buf: all of its 16 steps, or the first n
+    auto steps = [&](auto whole, auto buf_c, int k0, int n) {
+      constexpr int buf = decltype(buf_c)::value;
+      const float *ap = &As[buf][(wc * TC * 16 + c16) * FF_RS + 16 * h];
+      fp_f4 av[2][TC];  // the operands of this and the next 16 k
+#pragma unroll
+      for (int i = 0; i < TC; i++) av[0][i] = *(const fp_f4 *)(ap + i * 16 * FF_RS);
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        if (g < 3) {
+#pragma unroll
+          for (int i = 0; i < TC; i++) av[(g + 1) & 1][i] = *(const fp_f4 *)(ap + i * 16 * FF_RS + 4 * (g + 1));
+        }
+        float wk[TN][4];
+#pragma unroll
+        for (int t = 0; t < TN; t++) {
+          if constexpr (WH) {
+            const h2 lo = __builtin_bit_cast(h2, w[buf][t][g].x), hi = __builtin_bit_cast(h2, w[buf][t][g].y);
+            wk[t][0] = (float)lo.x, wk[t][1] = (float)lo.y, wk[t][2] = (float)hi.x, wk[t][3] = (float)hi.y;
+          } else {
+            wk[t][0] = w[buf][t][g].x, wk[t][1] = w[buf][t][g].y, wk[t][2] = w[buf][t][g].z, wk[t][3] = w[buf][t][g].w;
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+          if (decltype(whole)::value || 4 * g + s < n) {
+#pragma unroll
+            for (int i = 0; i < TC; i++)
+#pragma unroll
+              for (int t = 0; t < TN; t++)
+                acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[g & 1][i][s], wk[t][s], acc[i][t], 0, 0, 0);
+          }
+        if (decltype(whole)::value) fetch_w(buf, g, k0 + 2 * FF_KC);
+      }
+    };
+    std::integral_constant<int, 0> b0;
+    std::integral_constant<int, 1> b1;
+    __syncthreads();  // the previous cells' last reads of the buffers are done
+    fetch_a(0);
+#pragma unroll
+    for (int g = 0; g < 4; g++) fetch_w(0, g, 0);
+#pragma unroll
+    for (int g = 0; g < 4; g++) fetch_w(1, g, FF_KC);
+    commit_a(0);
     __syncthreads();
-    for (int k0 = 0, cur = 0; k0 < K; k0 += FP_KC, cur ^= 1) {
-      const bool more = k0 + FP_KC < K;
-      if (more) load(k0 + FP_KC);
-      const int kn = K - k0 < FP_KC ? K - k0 : FP_KC;  // 16 or 8 (K % 8 == 0)
-      for (int kk = 0; kk < kn; kk += 8) {
-#pragma unroll
-        for (int k = kk; k < kk + 8; k++) {
-          const float4 a0 = *(const float4 *)&As[cur][k][8 * cg], a1 = *(const float4 *)&As[cur][k][8 * cg + 4];
-          const float4 w0 = *(const float4 *)&Ws[cur][k][8 * pg], w1 = *(const float4 *)&Ws[cur][k][8 * pg + 4];
-          const float av[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-          const float wt[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-#pragma unroll
-          for (int i = 0; i < 8; i++)
-#pragma unroll
-            for (int j = 0; j < 8; j++) acc[i][j] = __builtin_fmaf(wt[j], av[i], acc[i][j]);
-        }
-      }
-      if (more) store(cur ^ 1);
+    int k0 = 0;
+    for (; K - k0 >= 2 * FF_KC; k0 += 2 * FF_KC) {
+      fetch_a(k0 + FF_KC);
+      steps(std::true_type{}, b0, k0, 16);
+      commit_a(1);
+      __syncthreads();
+      fetch_a(k0 + 2 * FF_KC);
+      steps(std::true_type{}, b1, k0 + FF_KC, 16);
+      commit_a(0);
       __syncthreads();
     }
+    // the chains stop at K (a multiple of 8)
+    if (K - k0 > FF_KC) {
+      fetch_a(k0 + FF_KC);
+      steps(std::true_type{}, b0, k0, 16);
+      commit_a(1);
+      __syncthreads();
+      steps(std::false_type{}, b1, 0, (K - k0 - FF_KC) / 4);
+    } else if (k0 < K) {
+      steps(std::false_type{}, b0, 0, (K - k0) / 4);
+    }
 #pragma unroll
-    for (int i = 0; i < 8; i++)
-      if (m0 + 8 * cg + i < P)
+    for (int i = 0; i < TC; i++)
 #pragma unroll
-        for (int j = 0; j < 8; j++) mx[j] = bnh_fmax(mx[j], acc[i][j]);
+      for (int t = 0; t < TN; t++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) mx[t] = bnh_fmax(mx[t], acc[i][t][j]);
   }
-  // the 8 cell groups of a prototype group are lanes l ^ 1, 2, 4
+  // lane (c, h) holds prototype c over a quarter of the cells of its wave
 #pragma unroll
-  for (int j = 0; j < 8; j++) {
-    mx[j] = bnh_fmax(mx[j], __shfl_xor(mx[j], 1));
-    mx[j] = bnh_fmax(mx[j], __shfl_xor(mx[j], 2));
-    mx[j] = bnh_fmax(mx[j], __shfl_xor(mx[j], 4));
+  for (int t = 0; t < TN; t++) {
+    mx[t] = bnh_fmax(mx[t], __shfl_xor(mx[t], 16));
+    mx[t] = bnh_fmax(mx[t], __shfl_xor(mx[t], 32));
   }
-  float v = mx[0];
+  if (WC > 1) {
+    __syncthreads();  // the last cells' reads are done
+    float *red = &As[0][0];  // [TN][WC][WN][16]
+    if (h == 0)
 #pragma unroll
-  for (int j = 1; j < 8; j++)
-    if (cg == j) v = mx[j];
-  const int n = n0 + 8 * pg + cg;
-  if (n < Np) colmax[win * cm_ws + n] = v;
+      for (int t = 0; t < TN; t++) red[((t * WC + wc) * WN + wn) * 16 + c16] = mx[t];
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < TN; t++)
+#pragma unroll
+      for (int q = 0; q < WC; q++) mx[t] = bnh_fmax(mx[t], red[((t * WC + q) * WN + wn) * 16 + c16]);
+  }
+#pragma unroll
+  for (int t = 0; t < TN; t++) {
+    const int n = (t0 + t) * 16 + c16;
+    if (wc == 0 && h == 0 && n < Np) colmax[win * cm_ws + n] = mx[t];
+  }
+}
+
+template <bool WH>
+static void ff_launch(const float *a, long long a_ws, int P, const bnh_fproto *W, float *colmax, long long cm_ws, int B,
+                      hipStream_t st) {
+  // The split with the least work on the fullest CU: its blocks there times the passes over the cells times a wave's
+  // step (TC TN matrix instructions and about half of one for its operands). 64 cells x 1536 against 5000 prototypes:
+  // 3 windows 4 cell tiles a wave 38 us, 2 by 2 waves 39, 1 by 4 waves 47 (281 us on the vector unit); one window 34, 23
+  // and 25; 4 windows 57, 51 and 52; 16 windows against 12,000 321, 351 and 435.
+  struct { int tc, wc, tn; } best = {4, 1, 1};
+  static const struct { int tc, wc, tn; } plan[] = {{4, 1, 2}, {3, 1, 2}, {2, 1, 2}, {4, 1, 1}, {3, 1, 1},
+                                                    {2, 1, 1}, {3, 2, 1}, {2, 2, 1}, {1, 2, 1}, {1, 4, 1}};
+  double least = 0;
+  for (const auto &p : plan) {
+    const long long blocks = B * bnh_ceil_div(W->Np, 16 * p.tn * (4 / p.wc));
+    const double cost = (double)bnh_ceil_div(blocks, 256) * bnh_ceil_div(P, 16 * p.tc * p.wc) * (p.tc * p.tn + 0.5);
+    if (least == 0 || cost < least) least = cost, best = {p.tc, p.wc, p.tn};
+  }
+#define FF_P(TC, WC, TN)                                                                                               \
+  if (best.tc == TC && best.wc == WC && best.tn == TN)                                                                 \
+  hipLaunchKernelGGL((k_colmax_f32<WH, TC, WC, TN>), dim3((unsigned)(B * bnh_ceil_div(W->Np, 16 * TN * (4 / WC)))),   \
+                     dim3(256), 0, st, a, a_ws, P, W->K, (const void *)W->w, W->Np, colmax, cm_ws, B)
+  FF_P(4, 1, 2);
+  FF_P(3, 1, 2);
+  FF_P(2, 1, 2);
+  FF_P(4, 1, 1);
+  FF_P(3, 1, 1);
+  FF_P(2, 1, 1);
+  FF_P(3, 2, 1);
+  FF_P(2, 2, 1);
+  FF_P(1, 2, 1);
+  FF_P(1, 4, 1);
+#undef FF_P
 }
 
 // ------------------------------------------------------------------ fp16 column maxima (kind 2)
@@ -314,7 +400,9 @@ bnh_fproto *bnh_fproto_new(int kind, int Np, int K, const void *w) {
     return nullptr;
   }
   const int Npt = (int)bnh_round_up(Np, FP_BN);
-  const size_t esz = kind == 0 ? 4 : 2, bytes = (size_t)K * Npt * esz;
+  const int K16 = (K + 15) / 16;
+  const size_t esz = kind == 0 ? 4 : 2;
+  const size_t bytes = (kind == 2 ? (size_t)K * Npt : (size_t)bnh_ceil_div(Np, 16) * K16 * 256) * esz;
   void *h = calloc(bytes, 1);
   bnh_fproto *W = (bnh_fproto *)calloc(1, sizeof *W);
   if (!h || !W) {
@@ -337,7 +425,9 @@ bnh_fproto *bnh_fproto_new(int kind, int Np, int K, const void *w) {
       step = 8;
     }
     for (int k = 0; k < K; k++) {
-      const size_t src = base + (size_t)k * step, dst = (size_t)k * Npt + n;
+      const size_t src = base + (size_t)k * step;
+      const size_t dst = kind == 2 ? (size_t)k * Npt + n
+                                   : (((size_t)(n / 16) * K16 + k / 16) * 64 + k % 4 * 16 + n % 16) * 4 + k % 16 / 4;
       if (esz == 4) ((float *)h)[dst] = ((const float *)w)[src];
       else ((uint16_t *)h)[dst] = ((const uint16_t *)w)[src];
     }
@@ -381,15 +471,21 @@ int bnh_fproto_colmax(const void *a, long long a_ws, int P, const bnh_fproto *W,
   const long long blocks = (long long)B * (W->Npt / FP_BN);
   BNH_REQ(blocks < (1LL << 31));
   if (B == 1) a_ws = cm_ws = 0;
-  if (W->kind == 2)
+  if (W->kind == 2) {
     hipLaunchKernelGGL(k_colmax_f16, dim3((unsigned)blocks), dim3(256), 0, bnh_stream(stream), (const uint16_t *)a, a_ws,
                        P, W->K, (const uint16_t *)W->w, W->Npt, W->Np, W->bs, W->nblk, colmax, cm_ws, B);
-  else if (W->kind == 1)
-    hipLaunchKernelGGL(k_colmax_f32<true>, dim3((unsigned)blocks), dim3(256), 0, bnh_stream(stream), (const float *)a,
-                       a_ws, P, W->K, (const void *)W->w, W->Npt, W->Np, colmax, cm_ws, B);
-  else
-    hipLaunchKernelGGL(k_colmax_f32<false>, dim3((unsigned)blocks), dim3(256), 0, bnh_stream(stream), (const float *)a,
-                       a_ws, P, W->K, (const void *)W->w, W->Npt, W->Np, colmax, cm_ws, B);
+  } else {
+    // windows per launch such that its tiles of 16 prototypes stay under 2^23 (a grid dimension is limited in threads)
+    const long long fit = (1LL << 23) / bnh_ceil_div(W->Np, 16);
+    const int most = fit < 1 ? 1 : fit > B ? B : (int)fit;
+    for (int b0 = 0; b0 < B; b0 += most) {
+      const int nb = B - b0 < most ? B - b0 : most;
+      const float *ab = (const float *)a + b0 * a_ws;
+      if (W->kind == 1) ff_launch<true>(ab, a_ws, P, W, colmax + b0 * cm_ws, cm_ws, nb, bnh_stream(stream));
+      else ff_launch<false>(ab, a_ws, P, W, colmax + b0 * cm_ws, cm_ws, nb, bnh_stream(stream));
+      BNH_HIP(hipGetLastError());
+    }
+  }
   BNH_HIP(hipGetLastError());
   return 0;
 }

@@ -73,6 +73,29 @@ def test_gemm_f32_shapes(hip, M, K, N, act):
         assert same(out[i], ref), ("window", i)
 
 
+@pytest.mark.parametrize("B,M,K,N,lda", [
+    (1, 1, 4, 8, 4), (1, 17, 28, 16, 28), (3, 5, 32, 24, 33), (2, 65, 36, 72, 38), (1, 6, 1396, 232, 1396),
+    (7, 33, 68, 40, 68), (40, 61, 64, 16, 64), (40, 61, 60, 32, 61), (40, 100, 132, 136, 132)])
+def test_gemm_f32_tiles(hip, B, M, K, N, lda):
+    """row lists that end inside a tile and tiles that span windows, every split of a block (few rows to many, one
+    channel tile to many), K at and beside the chunks of 32, rows that are not 16-byte aligned; values whose order of
+    summation shows: exponents over 2^40, sums and products in the denormal range"""
+    rng = np.random.default_rng(B * M + K + N)
+    w = np.ldexp(rng.standard_normal((N, K)), rng.integers(-20, 21, (N, K))).astype(np.float32)
+    w[: N // 4] = np.ldexp(rng.standard_normal((N // 4, K)), -70)
+    b = (rng.standard_normal(N) * 1e-40).astype(np.float32)
+    panels, bb, (_, _, Kp, Np) = netbuild.Net.fpack(w, b)
+    A = np.ldexp(rng.standard_normal((B, M, lda)), rng.integers(-20, 21, (B, M, lda))).astype(np.float32)
+    A[:, ::3] = np.ldexp(rng.standard_normal(A[:, ::3].shape), -68)
+    gate = rng.uniform(0, 1, (B, Kp)).astype(np.float32)
+    say("gemm_f32 tiles", B, M, K, N, lda)
+    for g in (None, gate):
+        out = run_gemm(hip, A, panels, bb, Kp, Np, gate=g, slack=24 if lda % 4 == 0 else 23)
+        for i in sorted({0, B // 2, B - 1}):
+            ref = O.gemm_f32(A[i], panels, bb, Kp, Np, gate=None if g is None else g[i])
+            assert same(out[i], ref), ("window", i)
+
+
 def test_gemm_f32_gate_residual_halo(hip):
     rng = np.random.default_rng(5)
     B, Hh, W, K, N = 2, 6, 10, 48, 40

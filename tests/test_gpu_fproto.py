@@ -105,6 +105,33 @@ def test_colmax(hip, kind, P, K, N, B):
         assert same(got[b], ref), (b, np.argwhere(got[b] != ref)[:4])
 
 
+@pytest.mark.parametrize("P,K,N,B", [(64, 72, 16, 1), (1, 64, 4104, 2), (16, 128, 1000, 40), (48, 56, 2048, 20),
+                                     (33, 200, 4100, 9), (96, 80, 1032, 3), (80, 64, 264, 30), (32, 8, 24, 3),
+                                     (65, 136, 6000, 1), (64, 40, 2056, 40)])
+def test_colmax_f32_splits(hip, P, K, N, B):
+    """each split of a block over cells and prototypes (one tile of cells to several passes, few prototypes to many),
+    ends inside tiles of 16; exponents over 2^30 and products in the denormal range, whose order of summation shows"""
+    H = hip
+    rng = np.random.default_rng(P * K + N + B)
+    protos = np.ldexp(rng.standard_normal((N, K)), rng.integers(-15, 16, (N, K))).astype(f32)
+    protos[::3] = np.ldexp(rng.standard_normal(protos[::3].shape), -75)
+    cells = np.ldexp(rng.standard_normal((B, P, K)), rng.integers(-15, 16, (B, P, K))).astype(f32)
+    cells[::2] = np.ldexp(rng.standard_normal(cells[::2].shape), -70)
+    for kind in ("f32", "f32h"):
+        p = protos if kind == "f32" else np.clip(protos, -60000, 60000)
+        w, Np = pack(kind, p)
+        Wd = H.FProto(KIND[kind], Np, K, w)
+        da = H.DeviceArray.from_host(cells)
+        dcm = H.DeviceArray.zeros((B, Np), f32)
+        say("fproto splits", kind, P, K, N, B)
+        H.check(H.lib().bnh_fproto_colmax(da.ptr, P * K, P, Wd.h, dcm.ptr, Np, B, None), "colmax")
+        H.sync()
+        got = dcm.numpy()
+        for b in sorted({0, B // 2, B - 1}):
+            ref = oracle_colmax(kind, cells[b], w, Np)
+            assert same(got[b], ref), (kind, b, np.argwhere(got[b] != ref)[:4])
+
+
 @pytest.mark.parametrize("kind", ["f32", "f32h", "f16"])
 def test_colmax_orders_and_specials(hip, kind):
     """rows whose chains the reference's order decides (absorption at 2^24 / fp16 2048, a fused product on -1),
