@@ -23,6 +23,7 @@
 
 #include <type_traits>
 
+#include "bnh_cells.h"
 #include "bnh_f16.h"
 #include "bnh_internal.h"
 #include "bnh_num.h"
@@ -35,42 +36,53 @@ struct bnh_fproto {
 };
 
 // ------------------------------------------------------------------ L2 normalisation of the cells
-// One wave per cell. The sum of squares is 8 fused chains (channel c feeds chain c % 8, in order of c: the two
-// 4-lane accumulators of 8-channel steps), combined as ((t0 + t1) + (t2 + t3)) with t_j = chain_j + chain_{j+4};
-// lanes 0..7 run the chains over a 512-float LDS chunk the whole wave stages. den = sqrtf(sum) + eps, a = x / den
-// (correctly rounded division); F16: fp16 cells widened, a rounded to fp16 (nearest even).
-#define L2_CHUNK 512
+// One wave per cell (bnh_cells.h). den = sqrtf(sum) + eps, a = x / den (correctly rounded division); F16: fp16 cells
+// widened, a rounded to fp16 (nearest even). vec, avec: the rows of x and of a are 16-byte (fp16: 8-byte) aligned.
 template <bool F16>
 __global__ __launch_bounds__(256) void k_l2norm(const void *__restrict__ xv, long long x_ws, int P, int C, int ld,
-                                                float eps, void *__restrict__ av, long long a_ws, long long cells) {
-  __shared__ float stage[4][L2_CHUNK];
+                                                float eps, void *__restrict__ av, long long a_ws, long long cells,
+                                                bool vec, bool avec) {
+  __shared__ __attribute__((aligned(16))) float stage[4][8 * CELL_LS];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const long long cell = (long long)blockIdx.x * 4 + wv;
+  long long cell = (long long)blockIdx.x * 4 + wv;
   const bool live = cell < cells;
-  const int w = live ? (int)(cell / P) : 0, p = live ? (int)(cell % P) : 0;
-  const float *r = F16 ? nullptr : (const float *)xv + w * x_ws + (long long)p * ld;
-  const h16 *rh = F16 ? (const h16 *)xv + w * x_ws + (long long)p * ld : nullptr;
+  if (!live) cell = cells - 1;
+  const long long w = cell / P;
+  const int p = (int)(cell - w * P);
+  const void *r = (const char *)xv + (w * x_ws + (long long)p * ld) * (F16 ? 2 : 4);
+  Cell x;
   float chain = 0.f;
-  for (int c0 = 0; c0 < C; c0 += L2_CHUNK) {
-    const int n = C - c0 < L2_CHUNK ? C - c0 : L2_CHUNK;
-    if (live)
-      for (int i = lane; i < n; i += 64) stage[wv][i] = F16 ? (float)rh[c0 + i] : r[c0 + i];
-    __syncthreads();
-    if (live && lane < 8)
-      for (int i = lane; i < n; i += 8) chain = __builtin_fmaf(stage[wv][i], stage[wv][i], chain);
-    __syncthreads();
+  for (int c0 = 0; c0 < C; c0 += CELL_CH) {
+    x.load<F16>(r, c0, C, vec, lane);
+    chain = x.squares(chain, C - c0 < CELL_CH ? C - c0 : CELL_CH, stage[wv], lane);
   }
   if (!live) return;
-  const float s1 = __shfl(chain, (lane & 3) + 4);
-  const float t = chain + s1;  // t_j in lanes 0..3
-  const float t0 = __shfl(t, 0), t1 = __shfl(t, 1), t2 = __shfl(t, 2), t3 = __shfl(t, 3);
-  const float den = __builtin_sqrtf((t0 + t1) + (t2 + t3)) + eps;
-  if (F16) {
-    h16 *a = (h16 *)av + w * a_ws + (long long)p * C;
-    for (int c = lane; c < C; c += 64) a[c] = f2h((float)rh[c] / den);
-  } else {
-    float *a = (float *)av + w * a_ws + (long long)p * C;
-    for (int c = lane; c < C; c += 64) a[c] = r[c] / den;
+  const float den = cell_norm(chain, lane) + eps;
+  const long long at = w * a_ws + (long long)p * C;
+  for (int c0 = 0; c0 < C; c0 += CELL_CH) {
+    if (C > CELL_CH) x.load<F16>(r, c0, C, vec, lane);
+#pragma unroll
+    for (int j = 0; j < CELL_CH / 256; j++) {
+      const int c = c0 + 256 * j + 4 * lane;
+      if (c >= C) continue;
+      const float4 y = make_float4(x.v[j].x / den, x.v[j].y / den, x.v[j].z / den, x.v[j].w / den);
+      if (F16) {
+        uint16_t *a = (uint16_t *)av + at + c;
+        const uint16_t e[4] = {hbits(f2h(y.x)), hbits(f2h(y.y)), hbits(f2h(y.z)), hbits(f2h(y.w))};
+        if (avec) {
+          *(uint2 *)a = make_uint2(e[0] | (uint32_t)e[1] << 16, e[2] | (uint32_t)e[3] << 16);
+        } else {
+          a[0] = e[0], a[1] = e[1], a[2] = e[2], a[3] = e[3];
+        }
+      } else {
+        float *a = (float *)av + at + c;
+        if (avec) {
+          *(float4 *)a = y;
+        } else {
+          a[0] = y.x, a[1] = y.y, a[2] = y.z, a[3] = y.w;
+        }
+      }
+    }
   }
 }
 
@@ -453,12 +465,15 @@ int bnh_l2norm_cells(const void *x, long long x_ws, int P, int C, int ld, float 
   BNH_REQ(C % 8 == 0 && ld >= C);
   BNH_REQ(B == 1 || (x_ws >= (long long)(P - 1) * ld + C && a_ws >= (long long)P * C));
   const long long cells = (long long)P * B;
+  const uintptr_t mask = f16 ? 7 : 15;
+  const bool vec = ((uintptr_t)x & mask) == 0 && ld % 4 == 0 && (B == 1 || x_ws % 4 == 0);
+  const bool avec = ((uintptr_t)a & mask) == 0 && (B == 1 || a_ws % 4 == 0);
   if (f16)
     hipLaunchKernelGGL(k_l2norm<true>, dim3((unsigned)bnh_ceil_div(cells, 4)), dim3(256), 0, bnh_stream(stream), x, x_ws,
-                       P, C, ld, eps, a, a_ws, cells);
+                       P, C, ld, eps, a, a_ws, cells, vec, avec);
   else
     hipLaunchKernelGGL(k_l2norm<false>, dim3((unsigned)bnh_ceil_div(cells, 4)), dim3(256), 0, bnh_stream(stream), x,
-                       x_ws, P, C, ld, eps, a, a_ws, cells);
+                       x_ws, P, C, ld, eps, a, a_ws, cells, vec, avec);
   BNH_HIP(hipGetLastError());
   return 0;
 }

@@ -9,6 +9,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include "bnh_cells.h"
 #include "bnh_internal.h"
 #include "bnh_lds_dma.h"
 #include "bnh_num.h"
@@ -27,62 +28,56 @@ static inline size_t s8p_at(int n, int k, int Kt) {
 }
 
 // ------------------------------------------------------------------ cell quantization (pc_quant_cells_f32)
-// One wave per cell. The reference's sum of squares is 8 fused chains (channel c feeds chain c % 8, in order of c):
-// lanes 0..7 run them over a 512-float LDS chunk the whole wave stages, then combine as ((t0 + t1) + (t2 + t3)),
-// t_j = chain_j + chain_{j+4}. max |x| (FMAX, NaN-propagating) is order-free: all lanes, then a wave reduction.
-#define QC_CHUNK 512
+// One wave per cell (bnh_cells.h). max |x| (FMAX, NaN-propagating) is order-free: all lanes, then a wave reduction.
 // F16: the cells are fp16 (pc_quant_cells_f16, src/pc_proto_s8.c:14-45: the same sums of the widened values, and
 // codes narrowed with saturation to [-128, 127] without the floor at -127)
 template <bool F16>
 __global__ __launch_bounds__(256) void k_quant_cells(const void *__restrict__ xv, long long x_ws, int P, int C, int ld,
                                                      float eps, int8_t *__restrict__ qa, long long qa_ws, int Kp,
-                                                     float *__restrict__ sx, long long sx_ws, long long cells) {
-  __shared__ float stage[4][QC_CHUNK];
+                                                     float *__restrict__ sx, long long sx_ws, long long cells,
+                                                     bool vec) {
+  __shared__ __attribute__((aligned(16))) float stage[4][8 * CELL_LS];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const long long cell = (long long)blockIdx.x * 4 + wv;
+  long long cell = (long long)blockIdx.x * 4 + wv;
   const bool live = cell < cells;
-  const int w = live ? (int)(cell / P) : 0, p = live ? (int)(cell % P) : 0;
-  const float *r = F16 ? nullptr : (const float *)xv + w * x_ws + (long long)p * ld;
-  const _Float16 *rh = F16 ? (const _Float16 *)xv + w * x_ws + (long long)p * ld : nullptr;
+  if (!live) cell = cells - 1;
+  const long long w = cell / P;
+  const int p = (int)(cell - w * P);
+  const void *r = (const char *)xv + (w * x_ws + (long long)p * ld) * (F16 ? 2 : 4);
+  Cell x;
   float chain = 0.f, mx = 0.f;
-  for (int c0 = 0; c0 < C; c0 += QC_CHUNK) {
-    const int n = C - c0 < QC_CHUNK ? C - c0 : QC_CHUNK;
-    if (live)
-      for (int i = lane; i < n; i += 64) {
-        const float v = F16 ? (float)rh[c0 + i] : r[c0 + i];
-        stage[wv][i] = v;
-        mx = bnh_fmax(mx, __builtin_fabsf(v));
-      }
-    __syncthreads();
-    if (live && lane < 8)
-      for (int i = lane; i < n; i += 8) chain = __builtin_fmaf(stage[wv][i], stage[wv][i], chain);
-    __syncthreads();
+  for (int c0 = 0; c0 < C; c0 += CELL_CH) {
+    x.load<F16>(r, c0, C, vec, lane);
+#pragma unroll
+    for (int j = 0; j < CELL_CH / 256; j++)
+      mx = bnh_fmax(bnh_fmax(bnh_fmax(mx, __builtin_fabsf(x.v[j].x)), __builtin_fabsf(x.v[j].y)),
+                    bnh_fmax(__builtin_fabsf(x.v[j].z), __builtin_fabsf(x.v[j].w)));
+    chain = x.squares(chain, C - c0 < CELL_CH ? C - c0 : CELL_CH, stage[wv], lane);
   }
   if (!live) return;
   for (int off = 32; off; off >>= 1) mx = bnh_fmax(mx, __shfl_xor(mx, off));
-  // lanes 0..3 hold chains j (channels 8i + j), lanes 4..7 chains j + 4: t_j = s0_j + s1_j
-  const float s1 = __shfl(chain, (lane & 3) + 4);
-  const float t = chain + s1;  // valid in lanes 0..3
-  const float t0 = __shfl(t, 0), t1 = __shfl(t, 1), t2 = __shfl(t, 2), t3 = __shfl(t, 3);
-  const float den = __builtin_sqrtf((t0 + t1) + (t2 + t3)) + eps;
+  const float den = cell_norm(chain, lane) + eps;
   if (!(mx > 0)) mx = 1e-30f;
   if (lane == 0) sx[w * sx_ws + p] = mx / (127.f * den);
   const float inv = 127.f / mx;
   int8_t *q = qa + w * qa_ws + (long long)p * Kp;
-  for (int c = lane * 4; c < Kp; c += 256) {
-    uint32_t word = 0;
+  for (int c0 = 0; c0 < Kp; c0 += CELL_CH) {
+    if (Kp > CELL_CH) x.load<F16>(r, c0, C, vec, lane);
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      int32_t b = 0;
-      if (c + j < C) {
-        int32_t v = bnh_cvta_s32((F16 ? (float)rh[c + j] : r[c + j]) * inv);
+    for (int j = 0; j < CELL_CH / 256; j++) {
+      const int c = c0 + 256 * j + 4 * lane;
+      if (c >= Kp) continue;
+      const float e[4] = {x.v[j].x, x.v[j].y, x.v[j].z, x.v[j].w};
+      uint32_t word = 0;
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        int32_t v = bnh_cvta_s32(e[u] * inv);
         v = v < -32768 ? -32768 : v > 32767 ? 32767 : v;
         v = v < -128 ? -128 : v > 127 ? 127 : v;
-        b = F16 || v >= -127 ? v : -127;
+        word |= ((uint32_t)(F16 || v >= -127 ? v : -127) & 0xffu) << (8 * u);
       }
-      word |= ((uint32_t)b & 0xffu) << (8 * j);
+      *(uint32_t *)(q + c) = c < C ? word : 0u;
     }
-    *(uint32_t *)(q + c) = word;
   }
 }
 
@@ -174,7 +169,7 @@ __global__ __launch_bounds__(256) void k_proto_colmax(const int8_t *__restrict__
 // K-blocked (see bnh_s8p), so each of their DMA instructions reads 1 KB of contiguous memory.
 //
 // Tile order: the tile grid (cell tiles x prototype tiles) is cut into 8 regions, one per XCD (blocks b, b + 8, ...
-// run on XCD b % 8), 8 x 1 when there are at least 8 cell tiles (each XCD's cells stay in its L2 while it streams every
+// run on XCD b % 8): 8 x 1 when there are at least 8 cell tiles (each XCD's cells stay in its L2 while it streams every
 // prototype once), fewer cell parts and more prototype parts for small batches. Within a region the tiles go
 // prototype-major, and the blocks of an XCD run through the same K slices at about the same time, so a slice one
 // block fetches is an L2 hit for the others.
@@ -583,8 +578,9 @@ int bnh_quant_cells(const float *x, long long x_ws, int P, int C, int ld, float 
   BNH_REQ(((uintptr_t)qa & 3) == 0 && qa_ws % 4 == 0);
   BNH_REQ(B == 1 || (qa_ws >= (long long)P * Kp && sx_ws >= P && x_ws >= (long long)(P - 1) * ld + C));
   const long long cells = (long long)P * B;
+  const bool vec = ((uintptr_t)x & 15) == 0 && ld % 4 == 0 && (B == 1 || x_ws % 4 == 0);
   hipLaunchKernelGGL(k_quant_cells<false>, dim3((unsigned)bnh_ceil_div(cells, 4)), dim3(256), 0, bnh_stream(stream), x,
-                     x_ws, P, C, ld, eps, qa, qa_ws, Kp, sx, sx_ws, cells);
+                     x_ws, P, C, ld, eps, qa, qa_ws, Kp, sx, sx_ws, cells, vec);
   BNH_HIP(hipGetLastError());
   return 0;
 }
@@ -596,8 +592,9 @@ int bnh_quant_cells_f16(const uint16_t *x, long long x_ws, int P, int C, int ld,
   BNH_REQ(((uintptr_t)qa & 3) == 0 && qa_ws % 4 == 0);
   BNH_REQ(B == 1 || (qa_ws >= (long long)P * Kp && sx_ws >= P && x_ws >= (long long)(P - 1) * ld + C));
   const long long cells = (long long)P * B;
+  const bool vec = ((uintptr_t)x & 7) == 0 && ld % 4 == 0 && (B == 1 || x_ws % 4 == 0);
   hipLaunchKernelGGL(k_quant_cells<true>, dim3((unsigned)bnh_ceil_div(cells, 4)), dim3(256), 0, bnh_stream(stream), x,
-                     x_ws, P, C, ld, eps, qa, qa_ws, Kp, sx, sx_ws, cells);
+                     x_ws, P, C, ld, eps, qa, qa_ws, Kp, sx, sx_ws, cells, vec);
   BNH_HIP(hipGetLastError());
   return 0;
 }

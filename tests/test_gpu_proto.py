@@ -54,7 +54,8 @@ def run_head(H, x, protos, clsw, clsb, nc, eps=1e-5):
 # (64, 256, ...) and (64, 512, ...) take the batched GEMM (64 cells per window, K in 64-byte slices); the others the
 # per-window kernel
 @pytest.mark.parametrize("P,C,N,nc", [(4, 8, 4, 1), (12, 48, 20, 5), (64, 136, 400, 100), (100, 96, 1000, 250),
-                                      (64, 256, 1000, 250), (64, 512, 2044, 511)])
+                                      (64, 256, 1000, 250), (64, 512, 2044, 511), (5, 2048, 12, 3), (9, 2056, 8, 2),
+                                      (4, 4160, 4, 1)])
 def test_head_small_shapes(hip, P, C, N, nc):
     rng = np.random.default_rng(P + C)
     B = 3
@@ -96,11 +97,11 @@ def test_head_perch_shape(hip):
         assert same(lg[b], rlg)
 
 
-@pytest.mark.parametrize("B", [5, 37])
+@pytest.mark.parametrize("B", [5, 20, 37])
 def test_batched_gemm_matches_per_window_kernel(hip, monkeypatch, B):
     """The batched column-max GEMM (tiles of 4 windows x 256 prototypes, split over the XCDs) against the
     one-window-per-block kernel on every window, and both against the oracle on some: B = 5 leaves a partial cell
-    tile and splits the prototypes over XCD regions, B = 37 gives 10 cell tiles over 8 regions."""
+    tile and splits the prototypes over XCD regions, B = 20 cuts 5 cell tiles, B = 37 gives 10 cell tiles over 8 regions."""
     H = hip
     rng = np.random.default_rng(40 + B)
     P, C, nc, ppc = 64, 1536, 1500, 4
