@@ -169,8 +169,7 @@ __global__ __launch_bounds__(256) void k_proto_colmax(const int8_t *__restrict__
 // K-blocked (see bnh_s8p), so each of their DMA instructions reads 1 KB of contiguous memory.
 //
 // Tile order: the tile grid (cell tiles x prototype tiles) is cut into 8 regions, one per XCD (blocks b, b + 8, ...
-// run on XCD b % 8): 8 x 1 when there are at least 8 cell tiles (each XCD's cells stay in its L2 while it streams every
-// prototype once), fewer cell parts and more prototype parts for small batches. Within a region the tiles go
+// run on XCD b % 8): gm parts of the cell tiles by 8 / gm of the prototype tiles, as the host chooses. Within a region the tiles go
 // prototype-major, and the blocks of an XCD run through the same K slices at about the same time, so a slice one
 // block fetches is an L2 hit for the others.
 //
@@ -219,7 +218,7 @@ struct PgRegion {
 __global__ __launch_bounds__(256, 1) void k_proto_gemm64(const int8_t *__restrict__ qa, long long qa_ws,
                                                         const float *__restrict__ sx, long long sx_ws, int B, int Kp,
                                                         const int8_t *__restrict__ wt, const float *__restrict__ sw,
-                                                        int Np, int n_mt, int n_nt, float *__restrict__ colmax,
+                                                        int Np, int n_mt, int n_nt, int gm, float *__restrict__ colmax,
                                                         long long cm_ws) {
   __shared__ __attribute__((aligned(1024))) int8_t lds_raw[PG_SCL + 2 * 2048];
   lds_i8 *lds = (lds_i8 *)lds_raw;
@@ -231,7 +230,7 @@ __global__ __launch_bounds__(256, 1) void k_proto_gemm64(const int8_t *__restric
   PgRegion R;
   R.lid = (int)(blockIdx.x >> 3);
   R.nlb = (int)(gridDim.x >> 3);
-  const int gm = n_mt >= 8 ? 8 : n_mt >= 4 ? 4 : n_mt >= 2 ? 2 : 1, gn = 8 / gm;
+  const int gn = 8 / gm;
   const int rm = xcd / gn, rn = xcd % gn;
   R.m_lo = rm * n_mt / gm;
   R.mx = (rm + 1) * n_mt / gm - R.m_lo;
@@ -372,7 +371,7 @@ BNH_DEV void pp_wait_next(int total, int s) {
 __global__ __launch_bounds__(512, 1) void k_proto_gemm_pp(const int8_t *__restrict__ qa, long long qa_ws,
                                                          const float *__restrict__ sx, long long sx_ws, int B, int Kp,
                                                          const int8_t *__restrict__ wt, const float *__restrict__ sw,
-                                                         int Np, int n_mt, int n_nt, float *__restrict__ colmax,
+                                                         int Np, int n_mt, int n_nt, int gm, float *__restrict__ colmax,
                                                          long long cm_ws) {
   __shared__ __attribute__((aligned(1024))) int8_t lds_raw[PG_SCL + 2 * 2048];
   lds_i8 *lds = (lds_i8 *)lds_raw;
@@ -383,7 +382,7 @@ __global__ __launch_bounds__(512, 1) void k_proto_gemm_pp(const int8_t *__restri
   PgRegion R;
   R.lid = (int)(blockIdx.x >> 3);
   R.nlb = (int)(gridDim.x >> 3);
-  const int gm = n_mt >= 8 ? 8 : n_mt >= 4 ? 4 : n_mt >= 2 ? 2 : 1, gn = 8 / gm;
+  const int gn = 8 / gm;
   const int rm = xcd / gn, rn = xcd % gn;
   R.m_lo = rm * n_mt / gm;
   R.mx = (rm + 1) * n_mt / gm - R.m_lo;
@@ -639,13 +638,28 @@ int bnh_proto_colmax(const int8_t *qa, long long qa_ws, const float *sx, long lo
     const int n_mt = (int)bnh_ceil_div((long long)B * 64, PG_TM), n_nt = W->Npt / PG_TN;
     int grid = ncu / 8 * 8;  // one block per CU
     if (grid < 8) grid = 8;
+    // The cut with the fewest tiles on the busiest block; among equals the one with more cell parts (each XCD's cells
+    // stay in its L2 while it streams its prototypes once). 20 windows, 5 cell tiles x 232 prototype tiles: in 4 x 2
+    // parts one XCD has two cell tiles and its blocks 8 tiles, in 1 x 8 every block has 4 or 5:
+    // the head 185 -> 127 us with the cells' faster quantization, 48 windows 311 -> 247, 70 windows 443 -> 356.
+    int gm = 1, least = 0;
+    for (int m = 1; m <= 8 && m <= n_mt; m *= 2) {
+      int most = 0;
+      for (int rm = 0; rm < m; rm++)
+        for (int rn = 0; rn < 8 / m; rn++) {
+          const int mx = (rm + 1) * n_mt / m - rm * n_mt / m, nx = (rn + 1) * n_nt / (8 / m) - rn * n_nt / (8 / m);
+          const int t = (int)bnh_ceil_div((long long)mx * nx, grid / 8);
+          if (t > most) most = t;
+        }
+      if (!least || most <= least) least = most, gm = m;
+    }
     static const bool four = getenv("BNH_PROTO_4W") != nullptr;  // the 4-wave form, for comparison
     if (four)
       hipLaunchKernelGGL(k_proto_gemm64, dim3((unsigned)grid), dim3(256), 0, bnh_stream(stream), qa, B == 1 ? 0 : qa_ws,
-                         sx, B == 1 ? 0 : sx_ws, B, W->Kp, W->w, W->sw, W->Np, n_mt, n_nt, colmax, B == 1 ? 0 : cm_ws);
+                         sx, B == 1 ? 0 : sx_ws, B, W->Kp, W->w, W->sw, W->Np, n_mt, n_nt, gm, colmax, B == 1 ? 0 : cm_ws);
     else
       hipLaunchKernelGGL(k_proto_gemm_pp, dim3((unsigned)grid), dim3(512), 0, bnh_stream(stream), qa, B == 1 ? 0 : qa_ws,
-                         sx, B == 1 ? 0 : sx_ws, B, W->Kp, W->w, W->sw, W->Np, n_mt, n_nt, colmax, B == 1 ? 0 : cm_ws);
+                         sx, B == 1 ? 0 : sx_ws, B, W->Kp, W->w, W->sw, W->Np, n_mt, n_nt, gm, colmax, B == 1 ? 0 : cm_ws);
     BNH_HIP(hipGetLastError());
     return 0;
   }
