@@ -39,6 +39,16 @@ struct bnh_s8w {
   int32_t *colsum;  // [Nt]
 };
 
+// bnh_pw_s8 without the halo zeroing (the halo is known to be zero); keep 0: the quantized rows, scales and zero points
+// may stay unwritten (nothing but this call's own GEMM reads them)
+extern "C" int bnh_pw_s8_body(const float *in, long long in_ws, int lda, int M, const float *gate, long long gate_ws,
+                              int8_t *q, long long q_ws, float *sa, long long sa_ws, int32_t *za, long long za_ws,
+                              int keep, int B, const bnh_s8w *W, const bnh_epi32 *e, void *stream);
+// bnh_pw_s8 whose workspace may stay unwritten
+extern "C" int bnh_pw_s8_scratch(const float *in, long long in_ws, int lda, int M, const float *gate, long long gate_ws,
+                                 int8_t *q, long long q_ws, float *sa, long long sa_ws, int32_t *za, long long za_ws,
+                                 int B, const bnh_s8w *W, const bnh_epi32 *e, void *stream);
+
 // whether bnh_pwdw_f32 takes this expansion + depthwise pair (0) or not (-1, with the reason in bnh_last_error)
 extern "C" int bnh_gemm_f16_mfma_body(const uint16_t *A, long long a_ws, int lda, int M, int B,
                                       const struct bnh_h16w *W, const bnh_epi16 *e, const uint16_t *gh,

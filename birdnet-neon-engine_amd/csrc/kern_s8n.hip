@@ -462,6 +462,287 @@ __global__ __launch_bounds__(256, 4) void k_s8n_gemm(const int8_t *__restrict__ 
   }
 }
 
+// ------------------------------------------------------------------ rows quantised by the block that multiplies them
+// bnh_pw_s8 as one launch: a block quantises its rows into LDS and multiplies them from there, so the int8 rows are
+// not written to memory, waited for and read back by a second launch (they are still written, once, for a caller
+// whose workspace keeps them). What bounds it: with many rows the fp32 rows' read from HBM, with few the latencies of
+// one row read, one weight read and the epilogue. The weights are the MFMA's first operand and the rows its second: a
+// lane then holds four neighbouring channels of one row, so residuals are read and outputs stored as 16-byte quads.
+// 16 rows a block: all their loads are in flight at once and five or more blocks share a CU (64 and 32 rows a block
+// read them in several round trips: 63 x 16 px x 40 windows, 288 -> 48, 33.7 and 29.8 us against 23.1).
+struct QRows {  // the rows to quantise, and where a caller's workspace keeps them (q NULL: nowhere)
+  const float *x;
+  long long x_ws;
+  int ld, M, K, Kp;
+  const float *gate;
+  long long g_ws;
+  int8_t *q;
+  long long q_ws;
+  float *sa;
+  long long sa_ws;
+  int32_t *za;
+  long long za_ws;
+  long long rows;
+  double rM;
+};
+
+// k_s8n_quant_v's quantisation (the same operations; K % 4 == 0, Kp <= 4 L QC) of the wave's RW rows, L lanes a row and
+// NR rows a lane at once, into LDS rows of S bytes; s_sa / s_z get the rows' scales and zero points
+template <int L, int QC, int NR, int RW>
+BNH_DEV void quant_rows_lds(const QRows &p, long long rowB, int lr0, bool keep, int8_t *A, int S, float *s_sa,
+                            uint32_t *s_z) {
+  constexpr int G = 64 / L;
+  static_assert(RW % (G * NR) == 0, "whole passes over the wave's rows");
+  const int lane = threadIdx.x & 63, sub = lane % L, n4 = p.K / 4, K8 = p.K & ~7;
+  for (int i0 = 0; i0 < RW; i0 += G * NR) {
+    float4 cv[NR][QC];
+    const float *r[NR], *g[NR];
+    int wi[NR], mi[NR];
+#pragma unroll
+    for (int a = 0; a < NR; a++) {
+      long long row = rowB + lr0 + i0 + a * G + lane / L;
+      row = row < p.rows ? row : p.rows - 1;
+      wi[a] = bnh_div(row, p.M, p.rM);
+      mi[a] = (int)(row - (long long)wi[a] * p.M);
+      r[a] = p.x + wi[a] * p.x_ws + (long long)mi[a] * p.ld;
+      g[a] = p.gate ? p.gate + wi[a] * p.g_ws : nullptr;
+#pragma unroll
+      for (int j = 0; j < QC; j++)
+        if (sub + j * L < n4) cv[a][j] = *(const float4 *)(r[a] + 4 * (sub + j * L));
+    }
+    // the NR rows' reductions side by side: one row's butterfly would wait on each of its exchanges
+    float lo[NR], hi[NR], inv[NR];
+    int32_t z[NR];
+    bool nan[NR], fast = true;
+#pragma unroll
+    for (int a = 0; a < NR; a++) {
+      int bad = 0;
+      lo[a] = __builtin_inff(), hi[a] = -__builtin_inff();
+#pragma unroll
+      for (int j = 0; j < QC; j++) {
+        if (sub + j * L >= n4) continue;
+        float4 &v = cv[a][j];
+        if (p.gate) {
+          const float4 gv = *(const float4 *)(g[a] + 4 * (sub + j * L));
+          v.x = v.x * gv.x; v.y = v.y * gv.y; v.z = v.z * gv.z; v.w = v.w * gv.w;
+        }
+        bad |= (v.x != v.x) | (v.y != v.y) | (v.z != v.z) | (v.w != v.w);
+        lo[a] = __builtin_fminf(__builtin_fminf(lo[a], v.x), __builtin_fminf(v.y, __builtin_fminf(v.z, v.w)));
+        hi[a] = __builtin_fmaxf(__builtin_fmaxf(hi[a], v.x), __builtin_fmaxf(v.y, __builtin_fmaxf(v.z, v.w)));
+      }
+      nan[a] = (__ballot(bad) >> (lane & ~(L - 1)) & (~0ull >> (64 - L))) != 0;  // in any lane of the row
+    }
+#pragma unroll
+    for (int off = L / 2; off; off >>= 1)
+#pragma unroll
+      for (int a = 0; a < NR; a++) {
+        lo[a] = __builtin_fminf(lo[a], __shfl_xor(lo[a], off));
+        hi[a] = __builtin_fmaxf(hi[a], __shfl_xor(hi[a], off));
+      }
+#pragma unroll
+    for (int a = 0; a < NR; a++) {
+      if (nan[a]) lo[a] = hi[a] = __builtin_nanf("");
+      float sc;
+      const float range = hi[a] - lo[a];
+      if (!(range > 1e-30f * bnh_fmaxnm(__builtin_fabsf(hi[a]), __builtin_fabsf(lo[a]))) || !(range > 0.f)) {
+        const float m = bnh_fmaxnm(__builtin_fabsf(hi[a]), 1e-30f);
+        inv[a] = 127.f / m;
+        z[a] = 0;
+        sc = m / 127.f;
+      } else {
+        inv[a] = 254.f / range;
+        z[a] = (int32_t)((uint32_t)-127 - (uint32_t)bnh_lrintf_s32(lo[a] * inv[a]));
+        sc = range / 254.f;
+      }
+      const int lr = lr0 + i0 + a * G + lane / L;
+      if (sub == 0) {
+        s_sa[lr] = sc;
+        s_z[lr] = (uint32_t)z[a];
+        if (keep && rowB + lr < p.rows) {
+          p.sa[wi[a] * p.sa_ws + mi[a]] = sc;
+          p.za[wi[a] * p.za_ws + mi[a]] = z[a];
+        }
+      }
+      fast &= !nan[a] && __builtin_fmaxf(__builtin_fabsf(lo[a]), __builtin_fabsf(hi[a])) * inv[a] < 1073741824.f;
+    }
+    auto store = [&](auto conv) {
+#pragma unroll
+      for (int a = 0; a < NR; a++) {
+        const int lr = lr0 + i0 + a * G + lane / L;
+        const bool kp = keep && rowB + lr < p.rows;
+        int8_t *o = A + lr * S, *og = p.q + wi[a] * p.q_ws + (long long)mi[a] * p.Kp;
+#pragma unroll
+        for (int j = 0; j < QC; j++) {
+          const int c = sub + j * L;
+          if (c >= p.Kp / 4) continue;
+          uint32_t word = ((uint32_t)z[a] & 0xffu) * 0x01010101u;  // past K: the zero point
+          if (c < n4) {
+            const float v[4] = {cv[a][j].x, cv[a][j].y, cv[a][j].z, cv[a][j].w};
+            word = 0;
+#pragma unroll
+            for (int jj = 0; jj < 4; jj++) {
+              int32_t cq = conv(v[jj] * inv[a], 4 * c, z[a]);
+              cq = cq < -127 ? -127 : cq > 127 ? 127 : cq;
+              word |= ((uint32_t)cq & 0xffu) << (8 * jj);
+            }
+          }
+          *(uint32_t *)(o + 4 * c) = word;
+          if (kp) *(uint32_t *)(og + 4 * c) = word;
+        }
+      }
+    };
+    if (__all(fast)) store([](float t, int, int32_t zz) { return (int32_t)__builtin_rintf(t) + zz; });
+    else
+      store([&](float t, int k, int32_t zz) {
+        return (int32_t)((uint32_t)(k < K8 ? bnh_cvtn_s32(t) : bnh_lrintf_s32(t)) + (uint32_t)zz);
+      });
+  }
+}
+
+struct QGemm {  // the multiplication, by value into the kernel
+  const int8_t *wt;
+  const float *sw;
+  const int32_t *cs;
+  const float *bias;
+  int Kp, Np, S;
+  EpiDev e;
+};
+
+// the epilogue of the lane's four channels n .. n + 3 of a row (k_s8n_gemm's operations), the residual quad added
+template <bool RES>
+BNH_DEV void qgemm_store(const QGemm &p, v4i acc, int n, float s_a, uint32_t z, float *out, const float4 &res,
+                         const uint32_t *tbl) {
+  const float4 sw = *(const float4 *)(p.sw + n), b = *(const float4 *)(p.bias + n);
+  const int4 cs = *(const int4 *)(p.cs + n);
+  const float swv[4] = {sw.x, sw.y, sw.z, sw.w}, bv[4] = {b.x, b.y, b.z, b.w}, rv[4] = {res.x, res.y, res.z, res.w};
+  const int csv[4] = {cs.x, cs.y, cs.z, cs.w};
+  float y[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int32_t c = (int32_t)((uint32_t)acc[r] - (uint32_t)csv[r] * z);
+    const float f = (float)c;
+    const float scl = swv[r] * s_a;
+    y[r] = f * scl;
+    y[r] = y[r] + bv[r];
+    if (p.e.act == 1) y[r] = bnh_silu_f32_t(y[r], tbl);
+    else if (p.e.act == 2) y[r] = bnh_relu_f32(y[r]);
+    if (RES) y[r] = y[r] + rv[r];
+  }
+  *(float4 *)(out + n) = make_float4(y[0], y[1], y[2], y[3]);
+}
+
+template <int R>
+BNH_DEV void qgemm_rows(const QRows &q, const QGemm &p, long long rowB, long long *s_o, long long *s_r) {
+  for (int i = threadIdx.x; i < R; i += 256) {
+    const long long row = rowB + i < q.rows ? rowB + i : q.rows - 1;
+    const int w = bnh_div(row, q.M, q.rM), m = (int)(row - (long long)w * q.M);
+    s_o[i] = w * p.e.out_ws + epi_prow(m, p.e.ow, p.e.opad, p.e.r_ow) * p.e.ldo;
+    s_r[i] = p.e.res ? w * p.e.res_ws + epi_prow(m, p.e.rw, p.e.rpad, p.e.r_rw) * p.e.ldr : 0;
+  }
+}
+
+// Many rows: a block owns 16 rows and every channel; each wave multiplies its share of the 16-channel tiles, two at a
+// time, the weights of four 64-byte K steps loaded together. With the SE gate and residual, 63 x 16 px: 288 -> 48,
+// 40 windows 28.9 -> 23.1 us (two launches -> this), 256 windows 138 -> 125 us; 32 x 8 px, 288 -> 96, 40 windows
+// 17.2 -> 10.1 us.
+template <int L, int QC, int NR, bool RES>
+__global__ __launch_bounds__(256, 4) void k_s8n_qgemm(QRows q, QGemm p) {
+  constexpr int R = 16, CT = 2, KC = 4;
+  __shared__ long long s_o[R], s_r[R];
+  __shared__ float s_sa[R];
+  __shared__ uint32_t s_z[R], s_tbl[256];
+  // R rows of S bytes and 64 more: a row's last K step may read past it
+  extern __shared__ __attribute__((aligned(16))) int8_t s_a8[];
+  if (p.e.act == 1) bnh_silu_table(s_tbl);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long long rowB = (long long)blockIdx.x * R;
+  qgemm_rows<R>(q, p, rowB, s_o, s_r);
+  quant_rows_lds<L, QC, NR, R / 4>(q, rowB, wave * (R / 4), q.q != nullptr, s_a8, p.S, s_sa, s_z);
+  __syncthreads();
+  const int nt = (p.Np + 15) / 16, kc = (lane >> 4) * 16, lr = lane & 15;
+  const int t1 = (wave + 1) * nt / 4, nst = (p.Kp + 63) / 64;
+  const int8_t *ap = s_a8 + lr * p.S + kc;
+  for (int t0 = wave * nt / 4; t0 < t1; t0 += CT) {
+    const int8_t *bp = p.wt + (long long)(16 * t0 + lr) * p.Kp + kc;
+    v4i acc[CT] = {(v4i){0, 0, 0, 0}, (v4i){0, 0, 0, 0}};
+    for (int s0 = 0; s0 < nst; s0 += KC) {
+      v4i b[KC][CT];
+#pragma unroll
+      for (int s = 0; s < KC; s++)
+#pragma unroll
+        for (int j = 0; j < CT; j++)  // zeros past Kp, whatever the row bytes there
+          b[s][j] = 64 * (s0 + s) + kc < p.Kp && t0 + j < t1 ? *(const v4i *)(bp + (long long)16 * j * p.Kp + 64 * (s0 + s))
+                                                             : (v4i){0, 0, 0, 0};
+#pragma unroll
+      for (int s = 0; s < KC; s++) {
+        if (s0 + s >= nst) break;
+        const v4i a = *(const v4i *)(ap + 64 * (s0 + s));
+#pragma unroll
+        for (int j = 0; j < CT; j++) acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(b[s][j], a, acc[j], 0, 0, 0);
+      }
+    }
+    float4 rq[CT];
+#pragma unroll
+    for (int j = 0; j < CT; j++) {
+      const int n = 16 * (t0 + j) + 4 * (lane >> 4);
+      rq[j] = RES && t0 + j < t1 && n < p.Np && rowB + lr < q.rows ? *(const float4 *)(p.e.res + s_r[lr] + n)
+                                                                  : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int j = 0; j < CT; j++) {
+      const int n = 16 * (t0 + j) + 4 * (lane >> 4);
+      if (t0 + j < t1 && n < p.Np && rowB + lr < q.rows)
+        qgemm_store<RES>(p, acc[j], n, s_sa[lr], s_z[lr], p.e.out + s_o[lr], rq[j], s_tbl);
+    }
+  }
+}
+
+// Few rows: a block owns 16 rows and 32 channels (parts blocks quantise the same rows), its waves a quarter of the K
+// steps each, all their weights loaded before the rows are quantised; the waves' int32 sums meet in LDS, in any order
+// the same. Kp <= 64 * 4 * KS. One window, two launches -> this: 63 x 16 px, 288 -> 48 13.8 -> 7.0 us; 16 x 4 px,
+// 1392 -> 232 24 -> 13.5 us; 1536 -> 14,795 over one row 19 -> 14.8 us.
+template <int L, int QC, int NR, int KS, bool RES>
+__global__ __launch_bounds__(256) void k_s8n_qgemm16(QRows q, QGemm p, int parts) {
+  constexpr int R = 16, CT = 2;
+  __shared__ long long s_o[R], s_r[R];
+  __shared__ float s_sa[R];
+  __shared__ uint32_t s_z[R], s_tbl[256];
+  __shared__ v4i s_acc[4][CT][64];
+  extern __shared__ __attribute__((aligned(16))) int8_t s_a8[];  // as above
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kc = (lane >> 4) * 16;
+  const long long rowB = (long long)(blockIdx.x / parts) * R;
+  const int part = blockIdx.x % parts, n0 = 32 * part, nst = (p.Kp + 63) / 64;
+  const int8_t *bp = p.wt + (long long)(n0 + (lane & 15)) * p.Kp + kc;
+  v4i b[KS][CT];
+#pragma unroll
+  for (int i = 0; i < KS; i++)
+#pragma unroll
+    for (int j = 0; j < CT; j++)
+      b[i][j] = 64 * (wave + 4 * i) + kc < p.Kp ? *(const v4i *)(bp + (long long)16 * j * p.Kp + 64 * (wave + 4 * i))
+                                                : (v4i){0, 0, 0, 0};
+  if (p.e.act == 1) bnh_silu_table(s_tbl);
+  qgemm_rows<R>(q, p, rowB, s_o, s_r);
+  quant_rows_lds<L, QC, NR, R / 4>(q, rowB, wave * (R / 4), q.q && part == 0, s_a8, p.S, s_sa, s_z);
+  __syncthreads();
+  const int8_t *ap = s_a8 + (lane & 15) * p.S + kc;
+  v4i acc[CT] = {(v4i){0, 0, 0, 0}, (v4i){0, 0, 0, 0}};
+#pragma unroll
+  for (int i = 0; i < KS; i++) {
+    if (wave + 4 * i >= nst) break;
+    const v4i a = *(const v4i *)(ap + 64 * (wave + 4 * i));
+#pragma unroll
+    for (int j = 0; j < CT; j++) acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(b[i][j], a, acc[j], 0, 0, 0);
+  }
+#pragma unroll
+  for (int j = 0; j < CT; j++) s_acc[wave][j][lane] = acc[j];
+  __syncthreads();
+  const int lr = lane & 15, n = n0 + 16 * wave + 4 * (lane >> 4);
+  if (wave >= CT || n >= p.Np || rowB + lr >= q.rows) return;
+  const v4i sum = s_acc[0][wave][lane] + s_acc[1][wave][lane] + s_acc[2][wave][lane] + s_acc[3][wave][lane];
+  const float4 rq = RES ? *(const float4 *)(p.e.res + s_r[lr] + n) : make_float4(0.f, 0.f, 0.f, 0.f);
+  qgemm_store<RES>(p, sum, n, s_sa[lr], s_z[lr], p.e.out + s_o[lr], rq, s_tbl);
+}
+
 // ------------------------------------------------------------------ int8 GEMM + fp32 dequant epilogue, large K
 // For Kp > 64 the per-group K loop of k_s8n_gemm re-reads a row's int8 bytes once per 64-channel group and waits on
 // every fragment load; here a block owns a tile of TR = 64 WM rows x TN = 128 WN channels (WM x WN = 4 waves, each
@@ -1441,6 +1722,21 @@ __global__ void k_eval_f32(int f, const float *__restrict__ x, float *__restrict
 }
 
 // ================================================================== host side
+static int check_quant(const float *x, long long x_ws, int ld, int M, int K, int Kp, const float *gate, const int8_t *q,
+                       long long q_ws, const float *sa, long long sa_ws, const int32_t *za, long long za_ws, int B) {
+  BNH_REQ(x && q && sa && za && M > 0 && K > 0 && B > 0);
+  BNH_REQ(Kp == ((K + 15) & ~15) && ld >= K);
+  BNH_REQ(!gate || (K % 4 == 0 && K <= 4096));
+  BNH_REQ(((uintptr_t)q & 3) == 0 && q_ws % 4 == 0 && (B == 1 || q_ws >= (long long)M * Kp));
+  BNH_REQ(B == 1 || (x_ws >= (long long)(M - 1) * ld + K && sa_ws >= M && za_ws >= M));
+  return 0;
+}
+// rows (and gates) that 16-byte loads may read
+static bool quant_vec(const float *x, long long x_ws, int ld, const float *gate, long long gate_ws, int B) {
+  return ((uintptr_t)x & 15) == 0 && ld % 4 == 0 && (B == 1 || x_ws % 4 == 0) &&
+         (!gate || (((uintptr_t)gate & 15) == 0 && (B == 1 || gate_ws % 4 == 0)));
+}
+
 extern "C" {
 
 int bnh_eval_requant(const int32_t *acc, const int32_t *mult, const int32_t *shift, int zy, int lo, int hi, int32_t *y,
@@ -1507,14 +1803,9 @@ void bnh_s8w_free(bnh_s8w *W) {
 int bnh_s8n_quant_rows(const float *x, long long x_ws, int ld, int M, int K, int Kp, const float *gate,
                        long long gate_ws, int8_t *q, long long q_ws, float *sa, long long sa_ws, int32_t *za,
                        long long za_ws, int B, void *stream) {
-  BNH_REQ(x && q && sa && za && M > 0 && K > 0 && B > 0);
-  BNH_REQ(Kp == ((K + 15) & ~15) && ld >= K);
-  BNH_REQ(!gate || (K % 4 == 0 && K <= 4096));
-  BNH_REQ(((uintptr_t)q & 3) == 0 && q_ws % 4 == 0 && (B == 1 || q_ws >= (long long)M * Kp));
-  BNH_REQ(B == 1 || (x_ws >= (long long)(M - 1) * ld + K && sa_ws >= M && za_ws >= M));
+  if (check_quant(x, x_ws, ld, M, K, Kp, gate, q, q_ws, sa, sa_ws, za, za_ws, B)) return -1;
   const long long rows = (long long)M * B;
-  const bool vec = ((uintptr_t)x & 15) == 0 && ld % 4 == 0 && (B == 1 || x_ws % 4 == 0) &&
-                   (!gate || (((uintptr_t)gate & 15) == 0 && (B == 1 || gate_ws % 4 == 0)));
+  const bool vec = quant_vec(x, x_ws, ld, gate, gate_ws, B);
   hipStream_t st = bnh_stream(stream);
   if (!vec) {
     hipLaunchKernelGGL(k_s8n_quant, dim3((unsigned)bnh_ceil_div(rows, 4)), dim3(256), 0, st, x, x_ws, ld, M, K, Kp,
@@ -1548,14 +1839,23 @@ static int check_epi(const bnh_epi32 *e, int M, int Np, int B) {
   return 0;
 }
 
-int bnh_s8n_gemm(const int8_t *q, long long q_ws, const float *sa, long long sa_ws, const int32_t *za, long long za_ws,
-                 int M, int B, const bnh_s8w *W, const bnh_epi32 *e, void *stream) {
+static EpiDev epi_dev(const bnh_epi32 *e) {
+  return {e->act, e->out, e->out_ws, e->ldo, e->ow, e->opad, e->res, e->res_ws, e->ldr, e->rpad, e->rw,
+          e->opad ? 1.0 / e->ow : 0.0, e->rpad ? 1.0 / e->rw : 0.0, 0};
+}
+static int check_gemm(const int8_t *q, long long q_ws, const float *sa, const int32_t *za, int M, int B, const bnh_s8w *W,
+                      const bnh_epi32 *e) {
   BNH_REQ(q && sa && za && W && M > 0 && B > 0);
   BNH_REQ(((uintptr_t)q & 15) == 0 && q_ws % 16 == 0);
   if (check_epi(e, M, W->Np, B)) return -1;
+  return 0;
+}
+
+int bnh_s8n_gemm(const int8_t *q, long long q_ws, const float *sa, long long sa_ws, const int32_t *za, long long za_ws,
+                 int M, int B, const bnh_s8w *W, const bnh_epi32 *e, void *stream) {
+  if (check_gemm(q, q_ws, sa, za, M, B, W, e)) return -1;
   const long long rows = (long long)M * B;
-  EpiDev d = {e->act, e->out, e->out_ws, e->ldo, e->ow, e->opad, e->res, e->res_ws, e->ldr, e->rpad, e->rw,
-              e->opad ? 1.0 / e->ow : 0.0, e->rpad ? 1.0 / e->rw : 0.0, 0};
+  EpiDev d = epi_dev(e);
   // with a residual, 16-byte quads when every output and residual quad lies 16-byte aligned (block 1's 24 -> 24
   // projection over 249 x 63 pixels 341 -> 322 us; without a residual the quads' LDS round trip made the launches
   // 10-30 % slower, so those store values directly)
@@ -1603,9 +1903,85 @@ int bnh_s8n_gemm(const int8_t *q, long long q_ws, const float *sa, long long sa_
   return 0;
 }
 
-int bnh_pw_s8(const float *in, long long in_ws, int lda, int M, const float *gate, long long gate_ws, int8_t *q,
-              long long q_ws, float *sa, long long sa_ws, int32_t *za, long long za_ws, int B, const bnh_s8w *W,
-              const bnh_epi32 *e, void *stream) {
+// pixel rows of a padded or plain image [first, one past the last] in floats from its base
+static long long epi_span(int M, int B, long long ws, int ld, int w, int pad) {
+  const long long rows = pad ? (long long)(M / w + 2 * pad) * (w + 2 * pad) : M;
+  return (B - 1) * (ws > 0 ? ws : 0) + rows * ld;
+}
+static bool overlap(const float *a, long long na, const float *b, long long nb) {
+  return (uintptr_t)a < (uintptr_t)(b + nb) && (uintptr_t)b < (uintptr_t)(a + na);
+}
+
+// the launch of k_s8n_qgemm or k_s8n_qgemm16 where they take the call: 1 launched, 0 not theirs, -1 an error
+static int qgemm_launch(const QRows &r, const bnh_s8w *W, const bnh_epi32 *e, int B, hipStream_t s) {
+  const int M = r.M, K = r.K, Kp = r.Kp;
+  auto al4 = [](const void *p, long long ws, int ld) { return ((uintptr_t)p & 15) == 0 && ws % 4 == 0 && ld % 4 == 0; };
+  if (!quant_vec(r.x, r.x_ws, r.ld, r.gate, r.g_ws, B) || K % 4 || Kp > 1536 || W->Np % 4) return 0;
+  if (!al4(e->out, e->out_ws, e->ldo) || (e->res && !al4(e->res, e->res_ws, e->ldr))) return 0;
+  // other blocks still read rows and gates when a block stores its outputs
+  const long long no = epi_span(M, B, e->out_ws, e->ldo, e->ow, e->opad);
+  if (r.x_ws < 0 || e->out_ws < 0 || r.g_ws < 0) return 0;
+  if (overlap(e->out, no, r.x, epi_span(M, B, r.x_ws, r.ld, 0, 0))) return 0;
+  if (r.gate && overlap(e->out, no, r.gate, (B - 1) * r.g_ws + K)) return 0;
+  QGemm p = {W->w, W->sw, W->colsum, W->b, Kp, W->Np, 16 * (Kp / 16 | 1), epi_dev(e)};  // odd: 16 rows, 16 bank groups
+  const int parts = (int)bnh_ceil_div(W->Np, 32);
+  const long long nb = bnh_ceil_div(r.rows, 16), few = nb * parts;
+  // Every channel of a row in one block: for 128 < Kp <= 512 and up to 128 channels at any number of rows (256 windows,
+  // 192 -> 32 over 125 x 32 px 312 -> 258 us; with K below, the two launches' wider blocks read rows faster: 24 -> 24
+  // over 249 x 63 px 304 against 554 us; with K above, the 16-row blocks re-read too many weights: 816 -> 136 over
+  // 32 x 8 px 130 against 157 us), and where the chip holds all blocks at once up to 256 channels whatever K (one
+  // window 24 -> 144 over 249 x 63 px 14.7 -> 9.3 us; 40 windows 1392 -> 232 over 16 x 4 px 30.9 -> 27.6 us;
+  // 1392 -> 384 32 against 34 us).
+  const bool whole = (Kp > 128 && Kp <= 512 && W->Np <= 128) || (W->Np <= 256 && nb <= 1024);
+  // The channels split over blocks while re-reading the rows costs less than the second launch: the lines lie between
+  // 3,328 blocks (136 -> 816, 15.1 -> 13.1 us) and 6,048 (192 -> 48, 23.4 against 25.2 us) for Kp <= 256, below
+  // 2,304 (288 -> 96, 18.3 against 19.8 us) for Kp <= 512, and past it, where two blocks fill a CU's registers, between
+  // 463 (19.1 -> 14.7 us) and 640 (576 -> 136, 16.6 against 19.7 us); for Kp <= 128 between 981 (11.5 -> 6.6 us) and
+  // 4,905 (14.7 against 15.5 us). Row blocks enough for every CU need no split (288 -> 96, 40 windows 17.9 against
+  // 10.1 us with whole rows), but for the shortest rows (981 blocks, 40 -> 24: 6.6 against 7.1 us).
+  const long long lim = Kp > 512 ? 512 : Kp > 256 ? 2048 : Kp > 128 ? 4096 : 2048;
+  if (few <= lim && !(whole && nb >= 256 && Kp > 128)) {
+#define QG(LL, QC, NR, KS)                                                                                       \
+  hipLaunchKernelGGL((e->res ? k_s8n_qgemm16<LL, QC, NR, KS, true> : k_s8n_qgemm16<LL, QC, NR, KS, false>),      \
+                     dim3((unsigned)few), dim3(256), 16 * p.S + 64, s, r, p, parts)
+    if (Kp <= 256) QG(16, 4, 1, 1);
+    else if (Kp <= 512) QG(32, 4, 2, 2);
+    else QG(64, 6, 4, 6);
+#undef QG
+  } else if (whole && nb < (1LL << 31)) {
+#define QG(LL, QC, NR)                                                                                \
+  hipLaunchKernelGGL((e->res ? k_s8n_qgemm<LL, QC, NR, true> : k_s8n_qgemm<LL, QC, NR, false>),       \
+                     dim3((unsigned)nb), dim3(256), 16 * p.S + 64, s, r, p)
+    if (Kp <= 128) QG(16, 2, 1);
+    else if (Kp <= 256) QG(16, 4, 1);
+    else if (Kp <= 512) QG(32, 4, 2);
+    else QG(64, 6, 2);
+#undef QG
+  } else
+    return 0;
+  BNH_HIP(hipGetLastError());
+  return 1;
+}
+
+int bnh_pw_s8_body(const float *in, long long in_ws, int lda, int M, const float *gate, long long gate_ws, int8_t *q,
+                   long long q_ws, float *sa, long long sa_ws, int32_t *za, long long za_ws, int keep, int B,
+                   const bnh_s8w *W, const bnh_epi32 *e, void *stream) {
+  BNH_REQ(W && e);
+  if (check_quant(in, in_ws, lda, M, W->K, W->Kp, gate, q, q_ws, sa, sa_ws, za, za_ws, B) ||
+      check_gemm(q, q_ws, sa, za, M, B, W, e))
+    return -1;
+  const QRows r = {in, in_ws, lda, M, W->K, W->Kp, gate, gate_ws, keep ? q : nullptr, q_ws, sa, sa_ws, za, za_ws,
+                   (long long)M * B, 1.0 / M};
+  const int f = qgemm_launch(r, W, e, B, bnh_stream(stream));
+  if (f) return f < 0 ? -1 : 0;
+  if (bnh_s8n_quant_rows(in, in_ws, lda, M, W->K, W->Kp, gate, gate_ws, q, q_ws, sa, sa_ws, za, za_ws, B, stream))
+    return -1;
+  return bnh_s8n_gemm(q, q_ws, sa, sa_ws, za, za_ws, M, B, W, e, stream);
+}
+
+static int pw_s8_run(const float *in, long long in_ws, int lda, int M, const float *gate, long long gate_ws, int8_t *q,
+                     long long q_ws, float *sa, long long sa_ws, int32_t *za, long long za_ws, int keep, int B,
+                     const bnh_s8w *W, const bnh_epi32 *e, void *stream) {
   BNH_REQ(W && e && e->out);
   if (check_epi(e, M, W->Np, B)) return -1;
   if (e->opad) {
@@ -1614,9 +1990,17 @@ int bnh_pw_s8(const float *in, long long in_ws, int lda, int M, const float *gat
     BNH_REQ(B == 1 || e->out_ws >= per);
     if (bnh_zero_halo(e->out, B == 1 ? per : e->out_ws, H, Wd, e->ldo, h, 4, B, stream)) return -1;
   }
-  if (bnh_s8n_quant_rows(in, in_ws, lda, M, W->K, W->Kp, gate, gate_ws, q, q_ws, sa, sa_ws, za, za_ws, B, stream))
-    return -1;
-  return bnh_s8n_gemm(q, q_ws, sa, sa_ws, za, za_ws, M, B, W, e, stream);
+  return bnh_pw_s8_body(in, in_ws, lda, M, gate, gate_ws, q, q_ws, sa, sa_ws, za, za_ws, keep, B, W, e, stream);
+}
+int bnh_pw_s8(const float *in, long long in_ws, int lda, int M, const float *gate, long long gate_ws, int8_t *q,
+              long long q_ws, float *sa, long long sa_ws, int32_t *za, long long za_ws, int B, const bnh_s8w *W,
+              const bnh_epi32 *e, void *stream) {
+  return pw_s8_run(in, in_ws, lda, M, gate, gate_ws, q, q_ws, sa, sa_ws, za, za_ws, 1, B, W, e, stream);
+}
+int bnh_pw_s8_scratch(const float *in, long long in_ws, int lda, int M, const float *gate, long long gate_ws, int8_t *q,
+                      long long q_ws, float *sa, long long sa_ws, int32_t *za, long long za_ws, int B, const bnh_s8w *W,
+                      const bnh_epi32 *e, void *stream) {
+  return pw_s8_run(in, in_ws, lda, M, gate, gate_ws, q, q_ws, sa, sa_ws, za, za_ws, 0, B, W, e, stream);
 }
 
 bnh_q8w *bnh_q8w_new(int N, int K, const int8_t *w, const int32_t *bias, const int32_t *mult, const int32_t *shift,

@@ -98,15 +98,12 @@ static int pw8_run(rt_ctx *c, rt_op *op) {
                  rt_ws(c, op, 2), p[10], r ? (int)r->halo : 0, r ? (int)r->W : 0};
   if (!e.opad) e.ow = 0;
   if (e.opad && rt_halo_kept(c, op, 1)) {  // the halo is still zero from the arena: quantize and multiply only
-    if (bnh_s8n_quant_rows((const float *)rt_b(c, op, 0), rt_ws(c, op, 0), p[5], p[4], p[1], p[2],
-                           gated ? (const float *)rt_b(c, op, 6) : nullptr, gated ? rt_ws(c, op, 6) : 0,
-                           (int8_t *)rt_b(c, op, 3), rt_ws(c, op, 3), (float *)rt_b(c, op, 4), rt_ws(c, op, 4),
-                           (int32_t *)rt_b(c, op, 5), rt_ws(c, op, 5), B, c->stream))
-      return -1;
-    return bnh_s8n_gemm((const int8_t *)rt_b(c, op, 3), rt_ws(c, op, 3), (const float *)rt_b(c, op, 4), rt_ws(c, op, 4),
-                        (const int32_t *)rt_b(c, op, 5), rt_ws(c, op, 5), p[4], B, s->W, &e, c->stream);
+    return bnh_pw_s8_body((const float *)rt_b(c, op, 0), rt_ws(c, op, 0), p[5], p[4],
+                          gated ? (const float *)rt_b(c, op, 6) : nullptr, gated ? rt_ws(c, op, 6) : 0,
+                          (int8_t *)rt_b(c, op, 3), rt_ws(c, op, 3), (float *)rt_b(c, op, 4), rt_ws(c, op, 4),
+                          (int32_t *)rt_b(c, op, 5), rt_ws(c, op, 5), 0, B, s->W, &e, c->stream);
   }
-  return bnh_pw_s8((const float *)rt_b(c, op, 0), rt_ws(c, op, 0), p[5], p[4],
+  return bnh_pw_s8_scratch((const float *)rt_b(c, op, 0), rt_ws(c, op, 0), p[5], p[4],
                    gated ? (const float *)rt_b(c, op, 6) : nullptr, gated ? rt_ws(c, op, 6) : 0, (int8_t *)rt_b(c, op, 3),
                    rt_ws(c, op, 3), (float *)rt_b(c, op, 4), rt_ws(c, op, 4), (int32_t *)rt_b(c, op, 5), rt_ws(c, op, 5), B,
                    s->W, &e, c->stream);
@@ -134,7 +131,7 @@ static int gemv8_run(rt_ctx *c, rt_op *op) {
   const s8_state *s = (const s8_state *)op->state;
   const int K = op->p[1], Np = op->p[3];
   bnh_epi32 e = {op->p[4], (float *)rt_b(c, op, 1), rt_ws(c, op, 1), Np, 0, 0, nullptr, 0, 0, 0, 0};
-  return bnh_pw_s8((const float *)rt_b(c, op, 0), rt_ws(c, op, 0), K, 1, nullptr, 0, (int8_t *)rt_b(c, op, 2),
+  return bnh_pw_s8_scratch((const float *)rt_b(c, op, 0), rt_ws(c, op, 0), K, 1, nullptr, 0, (int8_t *)rt_b(c, op, 2),
                    rt_ws(c, op, 2), (float *)rt_b(c, op, 3), rt_ws(c, op, 3), (int32_t *)rt_b(c, op, 4), rt_ws(c, op, 4),
                    c->nwin, s->W, &e, c->stream);
 }

@@ -64,5 +64,5 @@ extern "C" int bnh_pw_s8_static(const float *in, long long in_ws, int lda, int M
   float *sa = (float *)(base + qb);
   int32_t *za = (int32_t *)(base + qb + sb);
   const long long mk = (long long)M * W->Kp;
-  return bnh_pw_s8(in, in_ws, lda, M, gate, gate_ws, q, mk, sa, M, za, M, B, W, e, stream);
+  return bnh_pw_s8_scratch(in, in_ws, lda, M, gate, gate_ws, q, mk, sa, M, za, M, B, W, e, stream);
 }

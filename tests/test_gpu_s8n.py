@@ -157,7 +157,7 @@ def test_quant_rows_gate(hip):
 
 
 def pw_case(hip, B, H_, W_, K, N, act, opad=0, res=False, lda_extra=0, seed=0, gate=False, ldo_extra=8, rpad=0,
-            wins=None):
+            wins=None, edge=False):
     H = hip
     rng = np.random.default_rng(seed)
     M = H_ * W_
@@ -168,6 +168,12 @@ def pw_case(hip, B, H_, W_, K, N, act, opad=0, res=False, lda_extra=0, seed=0, g
     pk = s8pack.pack_s8(w, b)
     N_, K_, Kp, Np = pk["shape"]
     x = (rng.standard_normal((B, M, lda)) * 2).astype(np.float32)
+    if edge:  # constant, zero, far-offset, NaN, infinite and denormal rows
+        for i, v in enumerate((3.25, 0.0, 1e10, np.nan, np.inf, 1e-42)):
+            x[:, i % M, :K] = v if i < 2 else x[:, i % M, :K] + np.float32(v) if i == 2 else x[:, i % M, :K]
+            if i > 2:
+                x[:, i % M, (7 * i) % K] = v
+        x[-1, M - 1] *= np.float32(1e-42)
     gt = rng.uniform(0, 1, (B, K)).astype(np.float32) if gate else None
     ldo = Np + ldo_extra
     out_rows = M if not opad else (H_ + 2 * opad) * (W_ + 2 * opad)
@@ -254,6 +260,36 @@ def test_pw_s8_whole_k_steps(hip, K):
     """Rows that end exactly with a 64-wide K step (Kp 64, 128) and beside it, with and without a residual"""
     assert pw_case(hip, 2, 6, 11, K, 96, 1, seed=50 + K)
     assert pw_case(hip, 2, 6, 11, K, 24, 0, res=True, seed=60 + K)
+
+
+@pytest.mark.parametrize("K", [4, 60, 128, 132, 256, 260, 512, 516, 1020, 1536, 1540])
+def test_pw_s8_one_launch_rows(hip, K):
+    """Rows quantised by the block that multiplies them, at both sides of its K limits: few rows (channels split over
+    blocks; a lone row, a partial 16-row block) and more rows than that form takes (whole rows per block), partial
+    channel tiles, rows of special values, gate, haloed residual and output. Bytes of the int8 rows included."""
+    assert pw_case(hip, 1, 1, 1, K, 8, 0, seed=70 + K)
+    assert pw_case(hip, 3, 7, 9, K, 136, 1, opad=1, res=True, rpad=1, seed=71 + K, edge=True)
+    assert pw_case(hip, 2, 5, 6, K, 232, 2, seed=72 + K, gate=True, edge=True)
+    assert pw_case(hip, 3, 45, 41, K, 24, 0, res=True, gate=True, seed=73 + K, edge=True, wins=(0, 2))
+    if K in (132, 512):
+        assert pw_case(hip, 5, 45, 41, K, 120, 1, opad=1, seed=74 + K, wins=(4,))
+        assert pw_case(hip, 41, 45, 41, K, 24, 0, res=True, gate=True, seed=75 + K, wins=(0, 40))
+
+
+def test_pw_s8_output_over_its_input(hip):
+    """An output that takes its input's place: every row is quantised before any output is stored"""
+    H, rng = hip, np.random.default_rng(80)
+    M, K = 700, 144
+    pk = s8pack.pack_s8(rng.standard_normal((K, K)).astype(np.float32), rng.standard_normal(K).astype(np.float32))
+    Wt = H.S8Weights(K, K, K, K, pk["q"], pk["sw"], pk["cs"], pk["b"])
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    dx = H.DeviceArray.from_host(x)
+    dq, dsa, dza = H.DeviceArray.zeros((M, K), np.int8), H.DeviceArray.zeros(M, np.float32), H.DeviceArray.zeros(M, np.int32)
+    say("pw_s8 in place")
+    H.check(H.lib().bnh_pw_s8(dx.ptr, 0, K, M, None, 0, dq.ptr, 0, dsa.ptr, 0, dza.ptr, 0, 1, Wt.h,
+                              H.epi32(dx, K, act=1), None), "pw_s8")
+    H.sync()
+    assert same_f32(dx.numpy(), O.pw_s8(x, pk, act=1)[0][:, :K])
 
 
 def test_gemm_requant_config0(hip):
