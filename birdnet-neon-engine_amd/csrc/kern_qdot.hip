@@ -179,8 +179,12 @@ __global__ __launch_bounds__(256) void k_qd_quant(const void *__restrict__ xv, l
 // The same with L lanes per row (64 / L rows per wavefront) and 8 channels per lane per pass: 16-byte loads (fp16)
 // or two 16-byte loads (fp32), one 8-byte store of codes. K % 8 == 0, so every 8-channel chunk lies wholly in the
 // range part and wholly in the fp16 (or magic-number) code part or in the fp32 tail part; the lane group's range
-// reduction is order-free (NaN-propagating minima).
+// reduction is order-free. FMIN / FMAX give NaN when any value is NaN, which qd_params then takes for 0; plain minima
+// and maxima with a NaN flag give the same range (the sign of a zero extreme changes no parameter). The fp16 rows'
+// extremes and codes two channels an instruction: one by one they were most of the launch's vector work
+// (56 x 117 px x 64, gated, 12 windows).
 typedef _Float16 qv8h __attribute__((ext_vector_type(8)));
+typedef short qv8s __attribute__((ext_vector_type(8)));
 template <int L, bool F16>
 __global__ __launch_bounds__(256) void k_qd_quant_v(const void *__restrict__ xv, long long x_ws, int ldx, int M,
                                                     double rM, int K, int Kp, const uint16_t *__restrict__ gate,
@@ -196,30 +200,40 @@ __global__ __launch_bounds__(256) void k_qd_quant_v(const void *__restrict__ xv,
   const _Float16 *r16 = F16 ? (const _Float16 *)xv + w * x_ws + (long long)m * ldx : nullptr;
   const _Float16 *g = F16 && gate ? (const _Float16 *)gate + w * g_ws : nullptr;
   float mn = 0.f, mx = 0.f;
-  for (int c0 = 8 * sub; c0 < K; c0 += 8 * L) {
-    if (F16) {
+  int nan = 0;
+  if (F16) {
+    qv8h lo = (qv8h)(_Float16)0.f, hi = lo;
+    for (int c0 = 8 * sub; c0 < K; c0 += 8 * L) {
       qv8h h = *(const qv8h *)(r16 + c0);
       if (g) h = h * *(const qv8h *)(g + c0);
+      lo = __builtin_elementwise_min(lo, h);
+      hi = __builtin_elementwise_max(hi, h);
 #pragma unroll
-      for (int i = 0; i < 8; i++) {
-        mn = bnh_fmin(mn, (float)h[i]);
-        mx = bnh_fmax(mx, (float)h[i]);
-      }
-    } else {
+      for (int i = 0; i < 8; i++) nan |= h[i] != h[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      mn = __builtin_fminf(mn, (float)lo[i]);
+      mx = __builtin_fmaxf(mx, (float)hi[i]);
+    }
+  } else {
+    for (int c0 = 8 * sub; c0 < K; c0 += 8 * L) {
       const float4 u = *(const float4 *)(r32 + c0), v = *(const float4 *)(r32 + c0 + 4);
       const float e[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
 #pragma unroll
       for (int i = 0; i < 8; i++) {
-        mn = bnh_fmin(mn, e[i]);
-        mx = bnh_fmax(mx, e[i]);
+        nan |= e[i] != e[i];
+        mn = __builtin_fminf(mn, e[i]);
+        mx = __builtin_fmaxf(mx, e[i]);
       }
     }
   }
 #pragma unroll
   for (int off = 1; off < L; off <<= 1) {
-    mn = bnh_fmin(mn, __shfl_xor(mn, off));
-    mx = bnh_fmax(mx, __shfl_xor(mx, off));
+    mn = __builtin_fminf(mn, __shfl_xor(mn, off));
+    mx = __builtin_fmaxf(mx, __shfl_xor(mx, off));
   }
+  if (__ballot(nan) >> (lane & ~(L - 1)) & (~0ull >> (64 - L))) mn = mx = 0.f;  // in any lane of the row
   float s, zp, inv;
   qd_params(mn, mx, s, zp, inv);
   if (live && sub == 0) {
@@ -239,10 +253,12 @@ __global__ __launch_bounds__(256) void k_qd_quant_v(const void *__restrict__ xv,
         const qv8h gr = g ? *(const qv8h *)(g + c0) : (qv8h){};
         if (c0 < kq) {
           const qv8h h = g ? xr * gr : xr;  // the gated product rounded to fp16
-#pragma unroll
-          for (int i = 0; i < 8; i++)
-            (i < 4 ? lo : hi) |= (uint32_t)(uint8_t)qd_clamp8((int16_t)(uint16_t)(hbits(hfma(h[i], hinv, (h16)1536.0f)) -
-                                                                                    zo)) << (8 * (i & 3));
+          const qv8h t = __builtin_elementwise_fma(h, (qv8h)hinv, (qv8h)(_Float16)1536.0f);
+          qv8s q = __builtin_bit_cast(qv8s, t) - (qv8s)(short)zo;  // wrapping
+          q = __builtin_elementwise_min(__builtin_elementwise_max(q, (qv8s)(short)-128), (qv8s)(short)127);
+          const uint4 d = __builtin_bit_cast(uint4, q);
+          lo = __builtin_amdgcn_perm(d.y, d.x, 0x06040200u);
+          hi = __builtin_amdgcn_perm(d.w, d.z, 0x06040200u);
         } else {  // the fp32 tail: the unrounded product (exact in fp32), times the fp32 inv
 #pragma unroll
           for (int i = 0; i < 8; i++) {
@@ -285,19 +301,19 @@ struct QdConv {  // the 3 x 3 implicit im2col: A row m = output pixel (m / Wo, m
 // A block owns 128 rows; each wave 32 of them (2 MFMA row tiles) across the 64-channel groups [g0, g1) of its part.
 // CONV: k = 3 C ky + (kx C + c) over the haloed copy (its rows hold the 3 C bytes of kx = 0..2 contiguously), each
 // 16-byte chunk as two 8-byte halves, zero past 9 C.
-// VEC: each wave's 16 x 64 tile leaves the accumulators through LDS after its epilogue (the same operations, the
-// fp16 SiLU two values at a time from an LDS table) and is stored as 16-byte row chunks (fp32: the residual chunk
-// added to each), instead of one 2- or 4-byte store per value.
+// VEC: the weights are the MFMA's first operand and the rows its second, and tile j takes channels 16 q + 4 j + i
+// (q, i = 0..3) of the group: a lane's four tiles then hold 16 neighbouring channels of one row, which it activates
+// (the fp16 SiLU two values at a time from an LDS table) and stores as 16-byte chunks (fp32: the residual chunk added
+// to each), no LDS tile between.
 template <bool CONV, bool VEC>
-__global__ __launch_bounds__(256) void k_qd_gemm(const int8_t *__restrict__ a, long long a_ws, int lda,
+__global__ __launch_bounds__(256, 4) void k_qd_gemm(const int8_t *__restrict__ a, long long a_ws, int lda,
                                                  const float *__restrict__ rq, long long rq_ws, int per_tensor, int M,
                                                  double rM, long long rows, const int8_t *__restrict__ wt,
                                                  const float *__restrict__ sw, const float *__restrict__ sws,
                                                  const float *__restrict__ bias, int Kp, int Np, int gsplit, QdEpi e,
                                                  QdConv cv) {
-  constexpr int RB = 128, TS = 68;  // TS: the tile's LDS row stride in floats (64 channels + 4)
+  constexpr int RB = 128;
   __shared__ long long s_a[RB], s_o[RB], s_r[RB];
-  __shared__ __attribute__((aligned(16))) float s_t[VEC ? 4 : 1][VEC ? 16 * TS : 1];
   __shared__ uint32_t s_t01[16];
   __shared__ uint16_t s_t2[16];
   if (threadIdx.x < 16) {
@@ -334,7 +350,9 @@ __global__ __launch_bounds__(256) void k_qd_gemm(const int8_t *__restrict__ a, l
   for (int g = g0; g < g1; g++) {
     const int n0 = 64 * g;
     const int jn = Np - n0 >= 64 ? 4 : (Np - n0) / 16;  // Np % 16 == 0
-    const int8_t *bp = wt + (long long)(n0 + (lane & 15)) * Kp + kc;
+    // weight rows: tile j's channel of this lane is bc + bj j
+    const int bc = VEC ? 16 * ((lane & 15) >> 2) + (lane & 3) : lane & 15, bj = VEC ? 4 : 16;
+    const int8_t *bp = wt + (long long)(n0 + bc) * Kp + kc;
     v4i acc[2][4];
 #pragma unroll
     for (int t = 0; t < 2; t++)
@@ -363,14 +381,84 @@ __global__ __launch_bounds__(256) void k_qd_gemm(const int8_t *__restrict__ a, l
         }
       }
 #pragma unroll
-      for (int j = 0; j < 4; j++) bv[j] = kin && j < jn ? *(const v4i *)(bp + (long long)16 * j * Kp + k0) : (v4i){0, 0, 0, 0};
+      for (int j = 0; j < 4; j++)
+        bv[j] = kin && (VEC ? bc >> 4 : j) < jn ? *(const v4i *)(bp + (long long)bj * j * Kp + k0) : (v4i){0, 0, 0, 0};
 #pragma unroll
       for (int t = 0; t < 2; t++)
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-          if (j < jn) acc[t][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[t], bv[j], acc[t][j], 0, 0, 0);
+        for (int j = 0; j < 4; j++) {
+          if constexpr (VEC) acc[t][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bv[j], av[t], acc[t][j], 0, 0, 0);
+          else if (j < jn) acc[t][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[t], bv[j], acc[t][j], 0, 0, 0);
+        }
     }
     // epilogue (tile_row / affine4, src/gemm_s8.c:54-87,143-150)
+    if constexpr (VEC) {
+      if (lane >> 4 >= jn) continue;
+      const int n = n0 + 16 * (lane >> 4);
+      const int lr[2] = {lr0 + (lane & 15), lr0 + 16 + (lane & 15)};
+      const bool in[2] = {rowB + lr[0] < rows, rowB + lr[1] < rows};
+      const float sav[2] = {s_sa[lr[0]], s_sa[lr[1]]}, zsv[2] = {s_zs[lr[0]], s_zs[lr[1]]};
+      auto affine = [&](int t, int j, float v[4]) {
+        const float4 w4 = *(const float4 *)(sw + n + 4 * j), z4 = *(const float4 *)(sws + n + 4 * j);
+        const float4 b4 = *(const float4 *)(bias + n + 4 * j);
+        const float wv[4] = {w4.x, w4.y, w4.z, w4.w}, zv[4] = {z4.x, z4.y, z4.z, z4.w}, bb[4] = {b4.x, b4.y, b4.z, b4.w};
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const float v0 = (float)acc[t][j][r] * wv[r];
+          v[r] = __builtin_fmaf(zv[r], zsv[t], __builtin_fmaf(v0, sav[t], bb[r]));
+        }
+      };
+      if (e.out_f16) {
+        uint32_t h[2][8];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+          for (int t = 0; t < 2; t++) {
+            float v[4];
+            affine(t, j, v);
+#pragma unroll
+            for (int r = 0; r < 4; r += 2) {
+              h2 hv = (h2){f2h(v[r]), f2h(v[r + 1])};
+              if (e.act == 1) hv = silu2_lut(hv, s_t01, s_t2);
+              h[t][2 * j + r / 2] = __builtin_bit_cast(uint32_t, hv);
+            }
+          }
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+          if (!in[t]) continue;
+          uint4 *o = (uint4 *)((uint16_t *)e.out + s_o[lr[t]] + n);
+          o[0] = make_uint4(h[t][0], h[t][1], h[t][2], h[t][3]);
+          o[1] = make_uint4(h[t][4], h[t][5], h[t][6], h[t][7]);
+        }
+      } else {  // the residual chunks loaded before any store (out and res may alias)
+        float4 rv[2][4];
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+          for (int j = 0; j < 4; j++)
+            rv[t][j] = e.res && in[t] ? *(const float4 *)(e.res + s_r[lr[t]] + n + 4 * j) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+          for (int t = 0; t < 2; t++) {
+            float y[4];
+            affine(t, j, y);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+              if (e.act == 1) y[r] = qd_silu_f32_a(y[r]);
+              else if (e.act == 2) y[r] = bnh_relu_f32(y[r]);
+            }
+            if (e.res) {
+              y[0] = y[0] + rv[t][j].x;
+              y[1] = y[1] + rv[t][j].y;
+              y[2] = y[2] + rv[t][j].z;
+              y[3] = y[3] + rv[t][j].w;
+            }
+            if (in[t]) *(float4 *)((float *)e.out + s_o[lr[t]] + n + 4 * j) = make_float4(y[0], y[1], y[2], y[3]);
+          }
+      }
+      continue;
+    }
     float swn[4], ssn[4], bn[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
@@ -379,82 +467,6 @@ __global__ __launch_bounds__(256) void k_qd_gemm(const int8_t *__restrict__ a, l
       swn[j] = ok ? sw[n] : 0.f;
       ssn[j] = ok ? sws[n] : 0.f;
       bn[j] = ok ? bias[n] : 0.f;
-    }
-    if (VEC) {
-      float *T = s_t[wave];
-      const int nv = Np - n0 < 64 ? Np - n0 : 64;  // channels of this group (a multiple of 16)
-#pragma unroll
-      for (int t = 0; t < 2; t++) {
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          if (j >= jn) break;
-          float v[4];
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const int lr = lr0 + 16 * t + 4 * (lane >> 4) + r;
-            const float f = (float)acc[t][j][r];
-            const float v0 = f * swn[j];
-            v[r] = __builtin_fmaf(ssn[j], s_zs[lr], __builtin_fmaf(v0, s_sa[lr], bn[j]));
-          }
-          const int col = 16 * j + (lane & 15), rb = 4 * (lane >> 4);
-          if (e.out_f16) {
-            uint16_t *Th = (uint16_t *)T;  // [16][2 TS] halves
-#pragma unroll
-            for (int r = 0; r < 4; r += 2) {
-              h2 hv = (h2){f2h(v[r]), f2h(v[r + 1])};
-              if (e.act == 1) hv = silu2_lut(hv, s_t01, s_t2);
-              Th[(rb + r) * 2 * TS + col] = hbits(hv[0]);
-              Th[(rb + r + 1) * 2 * TS + col] = hbits(hv[1]);
-            }
-          } else {
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-              float y = v[r];
-              if (e.act == 1) y = qd_silu_f32_a(y);
-              else if (e.act == 2) y = bnh_relu_f32(y);
-              T[(rb + r) * TS + col] = y;
-            }
-          }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (e.out_f16) {  // 16 rows x 8 chunks of 8 halves: two per lane
-#pragma unroll
-          for (int it = 0; it < 2; it++) {
-            const int rr = 8 * it + (lane >> 3), ch = lane & 7, lr = lr0 + 16 * t + rr;
-            if (8 * ch < nv && rowB + lr < rows)
-              *(uint4 *)((uint16_t *)e.out + s_o[lr] + n0 + 8 * ch) =
-                  *(const uint4 *)((const uint16_t *)T + rr * 2 * TS + 8 * ch);
-          }
-        } else {  // 16 rows x 16 chunks of 4 floats: four per lane, the residual chunks loaded first
-          float4 rv4[4];
-#pragma unroll
-          for (int it = 0; it < 4; it++) {
-            const int rr = 4 * it + (lane >> 4), ch = lane & 15, lr = lr0 + 16 * t + rr;
-            rv4[it] = e.res && 4 * ch < nv && rowB + lr < rows ? *(const float4 *)(e.res + s_r[lr] + n0 + 4 * ch)
-                                                              : make_float4(0.f, 0.f, 0.f, 0.f);
-          }
-#pragma unroll
-          for (int it = 0; it < 4; it++) {
-            const int rr = 4 * it + (lane >> 4), ch = lane & 15, lr = lr0 + 16 * t + rr;
-            if (4 * ch < nv && rowB + lr < rows) {
-              float4 y = *(const float4 *)(T + rr * TS + 4 * ch);
-              if (e.res) {
-                y.x = y.x + rv4[it].x;
-                y.y = y.y + rv4[it].y;
-                y.z = y.z + rv4[it].z;
-                y.w = y.w + rv4[it].w;
-              }
-              *(float4 *)((float *)e.out + s_o[lr] + n0 + 4 * ch) = y;
-            }
-          }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      }
-      continue;
     }
 #pragma unroll
     for (int t = 0; t < 2; t++) {
