@@ -353,3 +353,29 @@ def test_mean_f16_and_gemv(hip):
     y = dy.numpy()
     for i in (0, 15, 16, 19):
         assert same_bits(y[i], O.gemv(w, b, xv[i], 0)), i
+
+
+@pytest.mark.parametrize("K,N,B,w16", [(8, 1, 1, 1), (24, 17, 2, 0), (32, 16, 16, 1), (40, 65, 17, 0), (136, 63, 33, 1),
+                                       (1032, 129, 5, 1), (24, 16389, 40, 1), (40, 16390, 35, 0)])
+def test_gemv_matrix_core_form(hip, K, N, B, w16):
+    """K % 8 == 0: partial steps of 32, partial output and window tiles, one and two window tiles a wave; sums that
+    underflow to -0, denormals, infinities and NaNs"""
+    H, rng = hip, np.random.default_rng(K * N + B)
+    w = (rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float16 if w16 else np.float32)
+    x = rng.standard_normal((B, K)).astype(np.float32)
+    w[N // 2] = -np.abs(w[N // 2])
+    x[B // 2] = np.abs(x[B // 2]) * np.float32(1e-43)
+    x[0, K - 1], x[B - 1, 3] = np.inf, np.nan
+    b = np.where(rng.random(N) < 0.5, 0.0, rng.standard_normal(N) * 0.1).astype(np.float32)
+    b[N // 2] = -0.0
+    dx, dw, db = H.DeviceArray.from_host(x), H.DeviceArray.from_host(w), H.DeviceArray.from_host(b)
+    dy = H.DeviceArray.from_host(np.full((B, N + 3), 9.0, np.float32))
+    say("gemv", K, N, B, w16)
+    H.check(H.lib().bnh_gemv(dw.ptr, w16, db.ptr, N, K, dx.ptr, K, 0, dy.ptr, N + 3, B, None), "gemv")
+    H.sync()
+    y = dy.numpy()
+    assert (y[:, N:] == 9.0).all()
+    for i in {0, B // 2, B - 1, min(B - 1, 31), min(B - 1, 32)}:
+        want = O.gemv(w, b, x[i], 0)
+        nan = np.isnan(want)
+        assert np.array_equal(np.isnan(y[i, :N]), nan) and same_bits(y[i, :N][~nan], want[~nan]), i
