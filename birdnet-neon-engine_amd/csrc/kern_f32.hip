@@ -398,13 +398,22 @@ __global__ __launch_bounds__(256) void k_se_scale(const float *__restrict__ gate
 }
 
 // ------------------------------------------------------------------ MEAN
+// 16 pixels' loads at once, then their sums in order (a load a sum waited on memory for each: 64 px x 1536 channels,
+// one window 16.7 -> 4.3 us)
 __global__ void k_mean_f32(const float *__restrict__ x, long long x_ws, int P, int C, int ld, float *__restrict__ out,
                            long long o_ws) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x, win = blockIdx.y;
   if (c >= C) return;
   const float *xw = x + win * x_ws + c;
   float s = 0.f;
-  for (int p = 0; p < P; p++) s = s + xw[(long long)p * ld];
+  for (int p = 0; p < P; p += 16) {
+    float v[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) v[u] = p + u < P ? xw[(long long)(p + u) * ld] : 0.f;
+#pragma unroll
+    for (int u = 0; u < 16; u++)
+      if (p + u < P) s = s + v[u];
+  }
   out[win * o_ws + c] = s / (float)P;
 }
 
@@ -415,7 +424,14 @@ __global__ void k_mean_f16(const uint16_t *__restrict__ x, long long x_ws, int P
   if (c >= C) return;
   const uint16_t *xw = x + win * x_ws + c;
   float s = 0.f;
-  for (int p = 0; p < P; p++) s = s + (float)hfrom(xw[(long long)p * ld]);
+  for (int p = 0; p < P; p += 16) {
+    float v[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) v[u] = p + u < P ? (float)hfrom(xw[(long long)(p + u) * ld]) : 0.f;
+#pragma unroll
+    for (int u = 0; u < 16; u++)
+      if (p + u < P) s = s + v[u];
+  }
   out[win * o_ws + c] = s / (float)P;
 }
 
