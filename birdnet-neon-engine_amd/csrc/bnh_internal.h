@@ -6,6 +6,7 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include "bnh_region.h"
 #include "bnneon_hip.h"
 
 // thread-local message of the kernel-level API (bnh_last_error)

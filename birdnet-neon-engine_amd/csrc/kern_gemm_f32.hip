@@ -213,14 +213,24 @@ extern "C" int bnh_gemm_f32(const float *A, long long a_ws, int lda, int M, cons
   double least = 0;
   static const struct { int tm, wm; } plan[] = {{4, 1}, {4, 2}, {2, 4}, {2, 1}, {2, 2}, {1, 4}, {1, 1}, {1, 2}};
   const long long all = (long long)M * B;
+  // An output over its input or gate: a row has to be read before anything is stored over it, which holds for blocks of
+  // 64 whole rows (Np <= 64; past its last barrier a block has read all it reads). Where each output row lies on its own
+  // input row they can all run at once; else the windows run one after the other, each its own block or blocks.
+  const bool rows_match = e->ldo == lda && !e->opad && (B == 1 || e->out_ws == a_ws);
+  const bnh_region so = bnh_windows(e->out, e->out_ws, bnh_rows_span(M, e->ldo, e->ow, e->opad));
+  const bool over_gate = gate && bnh_overlap(so, bnh_windows(gate, g_ws, Kp), B);
+  const bool over = over_gate || (bnh_overlap(so, bnh_windows(A, a_ws, bnh_rows_span(M, lda, 0, 0)), B) &&
+                                  !(rows_match && bnh_beside(A, Kp, (const float *)e->out, Np, lda)));
+  const bool at_once = !over || (!over_gate && rows_match && e->out == A);
   for (const auto &p : plan) {
+    if (over && least) break;  // the first of the list, 64 rows x 64 channels
     if (bnh_ceil_div(Np, 64 / p.wm) > 65535) continue;
     const long long blocks = bnh_ceil_div(all, 16 * p.tm * p.wm) * bnh_ceil_div(Np, 64 / p.wm);
     const double cost = (double)bnh_ceil_div(blocks, 256) * (p.tm + 0.5);
     if (least == 0 || cost < least) least = cost, best = {p.tm, p.wm};
   }
   // a launch takes at most 2^27 rows (a grid dimension is limited in threads)
-  const int most = (1 << 27) / M < 1 ? 1 : (1 << 27) / M;
+  const int most = !at_once || (1 << 27) / M < 1 ? 1 : (1 << 27) / M;
   for (int b0 = 0; b0 < B; b0 += most) {
     const int nb = B - b0 < most ? B - b0 : most;
     bnh_epi32 f = *e;

@@ -1903,15 +1903,6 @@ int bnh_s8n_gemm(const int8_t *q, long long q_ws, const float *sa, long long sa_
   return 0;
 }
 
-// pixel rows of a padded or plain image [first, one past the last] in floats from its base
-static long long epi_span(int M, int B, long long ws, int ld, int w, int pad) {
-  const long long rows = pad ? (long long)(M / w + 2 * pad) * (w + 2 * pad) : M;
-  return (B - 1) * (ws > 0 ? ws : 0) + rows * ld;
-}
-static bool overlap(const float *a, long long na, const float *b, long long nb) {
-  return (uintptr_t)a < (uintptr_t)(b + nb) && (uintptr_t)b < (uintptr_t)(a + na);
-}
-
 // the launch of k_s8n_qgemm or k_s8n_qgemm16 where they take the call: 1 launched, 0 not theirs, -1 an error
 static int qgemm_launch(const QRows &r, const bnh_s8w *W, const bnh_epi32 *e, int B, hipStream_t s) {
   const int M = r.M, K = r.K, Kp = r.Kp;
@@ -1919,10 +1910,9 @@ static int qgemm_launch(const QRows &r, const bnh_s8w *W, const bnh_epi32 *e, in
   if (!quant_vec(r.x, r.x_ws, r.ld, r.gate, r.g_ws, B) || K % 4 || Kp > 1536 || W->Np % 4) return 0;
   if (!al4(e->out, e->out_ws, e->ldo) || (e->res && !al4(e->res, e->res_ws, e->ldr))) return 0;
   // other blocks still read rows and gates when a block stores its outputs
-  const long long no = epi_span(M, B, e->out_ws, e->ldo, e->ow, e->opad);
-  if (r.x_ws < 0 || e->out_ws < 0 || r.g_ws < 0) return 0;
-  if (overlap(e->out, no, r.x, epi_span(M, B, r.x_ws, r.ld, 0, 0))) return 0;
-  if (r.gate && overlap(e->out, no, r.gate, (B - 1) * r.g_ws + K)) return 0;
+  const bnh_region so = bnh_windows(e->out, e->out_ws, bnh_rows_span(M, e->ldo, e->ow, e->opad));
+  if (bnh_overlap(so, bnh_windows(r.x, r.x_ws, bnh_rows_span(M, r.ld, 0, 0)), B)) return 0;
+  if (r.gate && bnh_overlap(so, bnh_windows(r.gate, r.g_ws, K), B)) return 0;
   QGemm p = {W->w, W->sw, W->colsum, W->b, Kp, W->Np, 16 * (Kp / 16 | 1), epi_dev(e)};  // odd: 16 rows, 16 bank groups
   const int parts = (int)bnh_ceil_div(W->Np, 32);
   const long long nb = bnh_ceil_div(r.rows, 16), few = nb * parts;

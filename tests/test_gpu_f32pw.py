@@ -96,6 +96,51 @@ def test_gemm_f32_tiles(hip, B, M, K, N, lda):
             assert same(out[i], ref), ("window", i)
 
 
+@pytest.mark.parametrize("B,M,K,N,ld,at", [
+    (5, 333, 48, 40, 48, 0), (1, 5000, 64, 64, 64, 0), (40, 61, 24, 16, 33, 0),   # each output row on its own input row
+    (3, 50, 32, 24, 40, 5), (9, 64, 16, 64, 72, -3),                              # M <= 64: a window's rows anywhere
+    (3, 200, 40, 24, 72, 44), (2, 150, 24, 136, 170, -140)])                      # columns beside the input's
+def test_gemm_f32_output_over_input(hip, B, M, K, N, ld, at):
+    """Outputs in their inputs' memory, `at` floats from the first input: a block's rows are read before any is stored"""
+    rng = np.random.default_rng(B * M + K + N)
+    w, b = rng.standard_normal((N, K)).astype(np.float32), rng.standard_normal(N).astype(np.float32)
+    panels, bb, (_, _, Kp, Np) = netbuild.Net.fpack(w, b)
+    first, ws = 160, M * ld + 320
+    buf = rng.standard_normal((B, ws)).astype(np.float32)
+    A = buf[:, first:first + M * ld].reshape(B, M, ld).copy()
+    d, dW, db = (hip.DeviceArray.from_host(v) for v in (buf, np.ascontiguousarray(panels), bb))
+    e = hip.Epi32(1, d.ptr + 4 * (first + at), ws, ld, 0, 0, None, 0, 0, 0, 0)
+    say("gemm_f32 over its input", B, M, K, N, ld, at)
+    hip.check(hip.lib().bnh_gemm_f32(d.ptr + 4 * first, ws, ld, M, None, 0, dW.ptr, db.ptr, Kp, Np, hip.C.byref(e), B,
+                                     None), "gemm_f32")
+    hip.sync()
+    got, want = d.numpy(), buf.copy()
+    for i in range(B):
+        rows = np.lib.stride_tricks.as_strided(want[i, first + at:], (M, N), (4 * ld, 4))
+        rows[:] = O.gemm_f32(A[i], panels, bb, Kp, Np, act=1)[:, :N]
+        assert same(got[i], want[i]), ("window", i)
+
+
+def test_gemm_f32_output_over_gate(hip):
+    """A gate in the memory of its window's outputs, M and Np within one block"""
+    rng = np.random.default_rng(9)
+    B, M, K, N = 7, 60, 48, 64
+    w, b = rng.standard_normal((N, K)).astype(np.float32), rng.standard_normal(N).astype(np.float32)
+    panels, bb, (_, _, Kp, Np) = netbuild.Net.fpack(w, b)
+    A, gate = rng.standard_normal((B, M, K)).astype(np.float32), rng.uniform(0, 1, (B, K)).astype(np.float32)
+    out = np.zeros((B, M * N), np.float32)
+    out[:, N:N + K] = gate
+    dA, do, dW, db = (hip.DeviceArray.from_host(v) for v in (A, out, np.ascontiguousarray(panels), bb))
+    e = hip.Epi32(0, do.ptr, M * N, N, 0, 0, None, 0, 0, 0, 0)
+    say("gemm_f32 over its gate")
+    hip.check(hip.lib().bnh_gemm_f32(dA.ptr, M * K, K, M, do.ptr + 4 * N, M * N, dW.ptr, db.ptr, Kp, Np,
+                                     hip.C.byref(e), B, None), "gemm_f32")
+    hip.sync()
+    got = do.numpy().reshape(B, M, N)
+    for i in range(B):
+        assert same(got[i], O.gemm_f32(A[i], panels, bb, Kp, Np, gate=gate[i])), ("window", i)
+
+
 def test_gemm_f32_gate_residual_halo(hip):
     rng = np.random.default_rng(5)
     B, Hh, W, K, N = 2, 6, 10, 48, 40
