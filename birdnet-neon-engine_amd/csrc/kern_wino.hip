@@ -593,10 +593,16 @@ int bnh_wino_f16(const uint16_t *x, long long x_ws, int H, int W, int ldx, const
     // with at most 32 input channels, whose blocks are small). The split with the least cost on the fullest CU: that
     // launch 20.7 us in 7 (22.4 in 6, 25.0 in 8), one window 82 -> 9.8 us in 24, 20 windows 84.5 -> 30 us in 3, and no
     // split from about 256 strips on (64 windows of 96 x 256 px: 122 us, 127 us in 2). Rows do not depend on the split.
+    // An output over its input (or a residual laid out otherwise): a strip's rows in order, each read before it is stored.
     const long long cols = (long long)strips * B;
+    const bnh_region so = bnh_windows(out, o_ws, bnh_rows_span(H * W, ldo, W, opad));
+    const bool own_res = res == out && rpad == opad && ldr == ldo && (B == 1 || r_ws == o_ws);
+    const bool over = bnh_overlap(so, bnh_windows(x, x_ws, bnh_rows_span(H * W, ldx, W, 1)), B) ||
+                      (res && !own_res && bnh_overlap(so, bnh_windows(res, r_ws, bnh_rows_span(H * W, ldr, W, rpad)), B));
+    const int most = over ? 1 : (H / 2 + 1) / 2;
     int nseg = 1;
     double least = 0;
-    for (int n = 1; n <= (H / 2 + 1) / 2 && (n == 1 || cols * n <= 2048); n++) {
+    for (int n = 1; n <= most && (n == 1 || cols * n <= 2048); n++) {
       const double cu = (double)bnh_ceil_div(cols * n, 256), share = nch == 1 ? 0.55 : 0.85;
       const double cost = (bnh_ceil_div(H / 2, n) + 2.5) * (cu > 1 ? share * cu : 1.0);
       if (n == 1 || cost < least) least = cost, nseg = n;

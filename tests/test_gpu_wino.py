@@ -125,6 +125,25 @@ def test_row_segments(hip, H, W, C, K, rpad):
     assert np.abs(plain - ref).max() <= 8 * 2.0 ** -11 * np.abs(ref).max()   # the whole-output bound used below
 
 
+@pytest.mark.parametrize("B,H,W,C", [(1, 62, 32, 64), (3, 40, 30, 24), (2, 96, 16, 40)])
+def test_output_over_its_input(hip, B, H, W, C):
+    """One strip a window (W <= 32), the output in its input's place: rows in order, each read before it is stored, and
+    the same bytes as into a buffer of its own"""
+    rng = np.random.default_rng(H + W + C)
+    xp, w, b = make(rng, B, H, W, C, C)
+    say("wino over its input", B, H, W, C)
+    want = run(hip, xp, w, b, act=1, opad=1)
+    P = hip.lib().bnh_wino16_new(C, C, w.ctypes.data, b.ctypes.data)
+    d = hip.DeviceArray.from_host(xp)
+    ws = (H + 2) * (W + 2) * C
+    try:
+        hip.check(hip.lib().bnh_wino_f16(d.ptr, ws, H, W, C, P, 1, d.ptr, ws, C, 1, None, 0, 0, 0, B, None), "wino_f16")
+        hip.sync()
+    finally:
+        hip.lib().bnh_wino16_free(P)
+    assert np.array_equal(d.numpy().view(np.uint16), want.view(np.uint16))
+
+
 def test_epilogue_forms(hip):
     rng = np.random.default_rng(3)
     B, H, W, C, K = 2, 6, 8, 16, 32
