@@ -339,8 +339,9 @@ __global__ __launch_bounds__(256, 2) void k_wino_f16r(const uint16_t *__restrict
   const int wi = __builtin_amdgcn_readfirstlane(tid >> 6);  // this wave's row of positions
   const int win = blockIdx.x / (strips * nseg), seg = blockIdx.x / strips % nseg, strip = blockIdx.x % strips;
   const int T = W / 2, tx0 = strip * WT_TILES, Wp = W + 2, c8 = C / 8;
-  const int S0 = (int)((long long)(H / 2) * seg / nseg);        // this block's tile rows [S0, NS)
-  const int NS = (int)((long long)(H / 2) * (seg + 1) / nseg);
+  const int per = H / 2 / nseg, more = H / 2 % nseg;  // tile rows of a segment, segments with one more
+  const int S0 = seg * per + (seg < more ? seg : more);
+  const int NS = S0 + per + (seg < more);  // this block's tile rows [S0, NS)
   const int ntl = T - tx0 < WT_TILES ? T - tx0 : WT_TILES;  // tiles of this strip that are stored
   // the window's haloed input as one buffer (columns past the image read the next row or zeros; tiles past T are
   // never stored)
@@ -591,8 +592,10 @@ int bnh_wino_f16(const uint16_t *x, long long x_ws, int H, int W, int ldx, const
     // so a strip's tile rows are split over nseg blocks. A block's cost is its rows + 2.5 (its U fragments and first
     // four input rows); blocks that share a CU each run slower: per block, k on a CU cost 0.85 k of one alone (0.55 k
     // with at most 32 input channels, whose blocks are small). The split with the least cost on the fullest CU: that
-    // launch 20.7 us in 7 (22.4 in 6, 25.0 in 8), one window 82 -> 9.8 us in 24, 20 windows 84.5 -> 30 us in 3, and no
-    // split from about 256 strips on (64 windows of 96 x 256 px: 122 us, 127 us in 2). Rows do not depend on the split.
+    // launch 20.7 us in 7 (22.4 in 6, 25.0 in 8), one window 82 -> 9.8 us in 24, 20 windows 84.5 -> 30 us in 3.
+    // From 257 strips on the unsplit blocks pair up too, and with more than 32 channels 0.85 prices the first pairs too
+    // high: two blocks run together in 1.25 of one's time (few such CUs) to 1.5 (all), a lone one behind them in 0.8 to
+    // 0.9. Priced so, the split has to beat the unsplit launch.
     // An output over its input (or a residual laid out otherwise): a strip's rows in order, each read before it is stored.
     const long long cols = (long long)strips * B;
     const bnh_region so = bnh_windows(out, o_ws, bnh_rows_span(H * W, ldo, W, opad));
@@ -607,6 +610,12 @@ int bnh_wino_f16(const uint16_t *x, long long x_ws, int H, int W, int ldx, const
       const double cost = (bnh_ceil_div(H / 2, n) + 2.5) * (cu > 1 ? share * cu : 1.0);
       if (n == 1 || cost < least) least = cost, nseg = n;
     }
+    auto paired = [&](int n) {
+      const double x = cols * n / 256.0, pairs = x > 1 ? ceil(x / 2) - 1 : 0, last = x - 2 * pairs;
+      const double load = x <= 1 ? 1.0 : 1.5 * pairs + (last > 1 ? 1.0 + 0.25 * last : 0.77 + 0.12 * last);
+      return (bnh_ceil_div(H / 2, n) + 2.5) * load;
+    };
+    if (nch > 1 && cols > 256 && paired(nseg) >= paired(1)) nseg = 1;
     const dim3 rgrid((unsigned)(cols * nseg));
 #define WINOR_A(NCH, NCB, ACT)                                                                                         \
   hipLaunchKernelGGL((k_wino_f16r<NCH, NCB, ACT>), rgrid, dim3(256), 0, st, x, x_ws, H, W, P->C, ldx, P->U, P->b,      \
