@@ -106,10 +106,10 @@ def test_within_stated_tolerance(hip, H, W, C, K):
                                           (94, 30, 32, 48, 1)])
 def test_row_segments(hip, H, W, C, K, rpad):
     """Few strips: each strip's tile rows are split over blocks (segments of two rows and more, uneven ones). The
-    rows do not depend on the split: one window and three equal the same windows of a batch long enough (260 strips
-    and more) to run unsplit, byte for byte, with a residual, SiLU and a zero halo"""
+    rows do not depend on the split: one window and three equal the same windows of a batch of more than 1024 strips,
+    which never splits, byte for byte, with a residual, SiLU and a zero halo"""
     rng = np.random.default_rng(H + W)
-    n = 260 // ((W // 2 + 15) // 16) + 1
+    n = 1024 // ((W // 2 + 15) // 16) + 1
     xp, w, b = make(rng, 3, H, W, C, K)
     res = np.zeros((3, H + 2 * rpad, W + 2 * rpad, K), np.float16)
     res[:] = rng.standard_normal(res.shape)
