@@ -815,7 +815,9 @@ int bnh_gemv(const void *w, int w16, const float *bias, int N, int K, const floa
   BNH_REQ(w && bias && x && out && N > 0 && K > 0 && B > 0 && (act == 0 || act == 2));
   BNH_REQ(B == 1 || (x_ws >= K && o_ws >= N));
   BNH_REQ((size_t)K * sizeof(float) <= 64 * 1024);
-  if (K % 8 == 0 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)x & 15) == 0 && (B == 1 || x_ws % 4 == 0)) {
+  // an output over its input: only the form below reads all of a window's input before it stores (N <= 32)
+  const bool over = bnh_overlap(bnh_windows(out, o_ws, N), bnh_windows(x, x_ws, K), B);
+  if (!over && K % 8 == 0 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)x & 15) == 0 && (B == 1 || x_ws % 4 == 0)) {
     // two window tiles a wave (each weight read serves both) once that leaves two waves for every SIMD
     const bool two = bnh_ceil_div(N, 16) * bnh_ceil_div(B, 32) >= 2048;
     const dim3 gm((unsigned)bnh_ceil_div(N, 64), (unsigned)bnh_ceil_div(B, two ? 32 : 16));

@@ -379,3 +379,19 @@ def test_gemv_matrix_core_form(hip, K, N, B, w16):
         want = O.gemv(w, b, x[i], 0)
         nan = np.isnan(want)
         assert np.array_equal(np.isnan(y[i, :N]), nan) and same_bits(y[i, :N][~nan], want[~nan]), i
+
+
+@pytest.mark.parametrize("K,N,B", [(32, 32, 1), (2048, 20, 40), (64, 31, 9)])
+def test_gemv_output_over_its_input(hip, K, N, B):
+    """N <= 32: a block has read all of its windows' inputs before it stores over them"""
+    H, rng = hip, np.random.default_rng(K + N + B)
+    w, b = rng.standard_normal((N, K)).astype(np.float32), rng.standard_normal(N).astype(np.float32)
+    x = rng.standard_normal((B, K)).astype(np.float32)
+    dx, dw, db = H.DeviceArray.from_host(x), H.DeviceArray.from_host(w), H.DeviceArray.from_host(b)
+    say("gemv over its input", K, N, B)
+    H.check(H.lib().bnh_gemv(dw.ptr, 0, db.ptr, N, K, dx.ptr, K, 2, dx.ptr, K, B, None), "gemv")
+    H.sync()
+    y = dx.numpy()
+    assert np.array_equal(y[:, N:], x[:, N:])
+    for i in range(B):
+        assert same_bits(y[i, :N], O.gemv(w, b, x[i], 2)), i
