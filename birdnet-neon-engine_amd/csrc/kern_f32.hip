@@ -815,9 +815,22 @@ int bnh_gemv(const void *w, int w16, const float *bias, int N, int K, const floa
   BNH_REQ(w && bias && x && out && N > 0 && K > 0 && B > 0 && (act == 0 || act == 2));
   BNH_REQ(B == 1 || (x_ws >= K && o_ws >= N));
   BNH_REQ((size_t)K * sizeof(float) <= 64 * 1024);
+  int wb = 8;
+  while (wb > 1 && (size_t)wb * K * sizeof(float) > 64 * 1024) wb /= 2;
   // an output over its input: only the form below reads all of a window's input before it stores (N <= 32)
   const bool over = bnh_overlap(bnh_windows(out, o_ws, N), bnh_windows(x, x_ws, K), B);
-  if (!over && K % 8 == 0 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)x & 15) == 0 && (B == 1 || x_ws % 4 == 0)) {
+  // The form below is the faster one for long rows while the chip holds all its blocks: past K 2048 it stages fewer than
+  // 8 windows a block, and a wave of the matrix form reads 32 rows some multiple of 16 KB apart. 1024 outputs x 4096, 8
+  // windows 35 against 49 us (fp16 weights 32, 45), x 8192, 32 windows 90, 114 (45, 88); with more blocks (1024 x 8192, 48
+  // windows) 178, 114 (87, 88). Wide layers are bound by reading their weights, which the matrix form does once for 16
+  // windows: 6522 x 4096, 2 windows 54, 63 (52, 53) and 8 windows 71, 51 (67, 54); 14795 x 8192, one 169, 145 (87, 99).
+  const long long blocks = bnh_ceil_div(N, 32) * bnh_ceil_div(B, wb);
+  const bool long_rows = K > 2048 && blocks <= 512 && (N <= 4096 || (N <= 8192 && B <= 2));
+  // And for one or two windows of middling fp16 layers, by 3 to 6 %: 1024 x 1024, one window 13.9 against 14.7 us, 6522 x
+  // 1024 14.1, 14.7; not 1024 x 64 (4.2, 3.9), 6522 x 2048 (32, 27) nor four windows (16, 15).
+  const bool lone = w16 && B <= 2 && K >= 512 && K * B <= 2048 && N >= 128 && N <= 8192 && (long long)N * K <= 8 << 20;
+  if (!over && !long_rows && !lone && K % 8 == 0 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)x & 15) == 0 &&
+      (B == 1 || x_ws % 4 == 0)) {
     // two window tiles a wave (each weight read serves both) once that leaves two waves for every SIMD
     const bool two = bnh_ceil_div(N, 16) * bnh_ceil_div(B, 32) >= 2048;
     const dim3 gm((unsigned)bnh_ceil_div(N, 64), (unsigned)bnh_ceil_div(B, two ? 32 : 16));
@@ -826,8 +839,6 @@ int bnh_gemv(const void *w, int w16, const float *bias, int N, int K, const floa
     BNH_HIP(hipGetLastError());
     return 0;
   }
-  int wb = 8;
-  while (wb > 1 && (size_t)wb * K * sizeof(float) > 64 * 1024) wb /= 2;
   const dim3 grid((unsigned)bnh_ceil_div(N, 32), (unsigned)bnh_ceil_div(B, wb));
   const size_t lds = sizeof(float) * (size_t)wb * K;
   hipStream_t st = bnh_stream(stream);

@@ -381,6 +381,24 @@ def test_gemv_matrix_core_form(hip, K, N, B, w16):
         assert np.array_equal(np.isnan(y[i, :N]), nan) and same_bits(y[i, :N][~nan], want[~nan]), i
 
 
+@pytest.mark.parametrize("K,N,B,w16", [(2048, 40, 9, 0), (2056, 40, 9, 0), (4096, 16, 2048, 1), (4096, 16, 2049, 1),
+                                       (2064, 4100, 3, 0), (2064, 4100, 2, 1), (512, 128, 2, 1), (1024, 127, 2, 1),
+                                       (1032, 130, 2, 1), (504, 130, 1, 1)])
+def test_gemv_form_limits(hip, K, N, B, w16):
+    """Both sides of each line between the two forms: long rows, their block count, wide layers, one or two windows"""
+    H, rng = hip, np.random.default_rng(K * N + B)
+    w = (rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float16 if w16 else np.float32)
+    x, b = rng.standard_normal((B, K)).astype(np.float32), rng.standard_normal(N).astype(np.float32)
+    dx, dw, db = H.DeviceArray.from_host(x), H.DeviceArray.from_host(w), H.DeviceArray.from_host(b)
+    dy = H.DeviceArray.zeros((B, N), np.float32)
+    say("gemv forms", K, N, B, w16)
+    H.check(H.lib().bnh_gemv(dw.ptr, w16, db.ptr, N, K, dx.ptr, K, 2, dy.ptr, N, B, None), "gemv")
+    H.sync()
+    y = dy.numpy()
+    for i in {0, B // 2, B - 1}:
+        assert same_bits(y[i], O.gemv(w, b, x[i], 2)), i
+
+
 @pytest.mark.parametrize("K,N,B", [(32, 32, 1), (2048, 20, 40), (64, 31, 9)])
 def test_gemv_output_over_its_input(hip, K, N, B):
     """N <= 32: a block has read all of its windows' inputs before it stores over them"""
