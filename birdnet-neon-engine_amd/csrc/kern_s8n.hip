@@ -1913,6 +1913,14 @@ static int qgemm_launch(const QRows &r, const bnh_s8w *W, const bnh_epi32 *e, in
   const bnh_region so = bnh_windows(e->out, e->out_ws, bnh_rows_span(M, e->ldo, e->ow, e->opad));
   if (bnh_overlap(so, bnh_windows(r.x, r.x_ws, bnh_rows_span(M, r.ld, 0, 0)), B)) return 0;
   if (r.gate && bnh_overlap(so, bnh_windows(r.gate, r.g_ws, K), B)) return 0;
+  if (r.q) {  // and the kept workspace is written by some blocks while others read their inputs and store outputs
+    const bnh_region kept[3] = {bnh_windows(r.q, r.q_ws, (long long)M * Kp), bnh_windows(r.sa, r.sa_ws, M),
+                                bnh_windows(r.za, r.za_ws, M)};
+    for (const bnh_region &k : kept)
+      if (bnh_overlap(k, so, B) || bnh_overlap(k, bnh_windows(r.x, r.x_ws, bnh_rows_span(M, r.ld, 0, 0)), B) ||
+          (r.gate && bnh_overlap(k, bnh_windows(r.gate, r.g_ws, K), B)))
+        return 0;
+  }
   QGemm p = {W->w, W->sw, W->colsum, W->b, Kp, W->Np, 16 * (Kp / 16 | 1), epi_dev(e)};  // odd: 16 rows, 16 bank groups
   const int parts = (int)bnh_ceil_div(W->Np, 32);
   const long long nb = bnh_ceil_div(r.rows, 16), few = nb * parts;

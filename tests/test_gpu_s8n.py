@@ -292,6 +292,26 @@ def test_pw_s8_output_over_its_input(hip):
     assert same_f32(dx.numpy(), O.pw_s8(x, pk, act=1)[0][:, :K])
 
 
+def test_pw_s8_workspace_over_its_row(hip):
+    """One row whose int8 codes, scale and zero point are kept in the memory it was read from: every channel's sum is of
+    the row as it was"""
+    H, rng = hip, np.random.default_rng(81)
+    K, N = 288, 400
+    pk = s8pack.pack_s8(rng.standard_normal((N, K)).astype(np.float32), rng.standard_normal(N).astype(np.float32))
+    Wt = H.S8Weights(N, K, K, N, pk["q"], pk["sw"], pk["cs"], pk["b"])
+    x = rng.standard_normal((1, K)).astype(np.float32)
+    dx, dout = H.DeviceArray.from_host(x), H.DeviceArray.zeros((1, N), np.float32)
+    say("pw_s8 workspace over its row")
+    H.check(H.lib().bnh_pw_s8(dx.ptr, 0, K, 1, None, 0, dx.ptr, 0, dx.ptr + K, 0, dx.ptr + K + 4, 0, 1, Wt.h,
+                              H.epi32(dout, N, act=1), None), "pw_s8")
+    H.sync()
+    want, rq, rsa, rza = O.pw_s8(x, pk, act=1)
+    got = dx.numpy().view(np.uint8)[0]
+    assert same_f32(dout.numpy(), want[:, :N])
+    assert np.array_equal(got[:K].view(np.int8), rq[0, :K])
+    assert got[K:K + 4].view(np.float32)[0] == rsa[0] and got[K + 4:K + 8].view(np.int32)[0] == rza[0]
+
+
 def test_gemm_requant_config0(hip):
     H = hip
     rng = np.random.default_rng(2024)
