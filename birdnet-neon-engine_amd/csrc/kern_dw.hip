@@ -976,8 +976,12 @@ static int chsum_launch(const T *out, long long o_ws, int C, int Ho, int Wo, flo
     constexpr int S = decltype(s_)::value, most = CsPlan<FORM, S>::TT;
     const int TT = NT < most ? (int)bnh_round_up(NT, 4) : most, slabs = (int)bnh_ceil_div(C, S);
     const size_t lds = 4 * ((size_t)(NT > TT ? 2 : 1) * S * (TT + 4) + 16);
-    hipLaunchKernelGGL((k_chsum<T, FORM, S>), dim3((unsigned)((long long)slabs * B)), dim3(256), lds, st, out, o_ws, C,
-                       Wo, NT, TT, slabs, 1.0 / Tn, chsum, cs_ws);
+    const int wins = (1 << 23) / slabs < 1 ? 1 : (1 << 23) / slabs;  // windows a launch: 2^32 threads are too many
+    for (long long b0 = 0; b0 < B; b0 += wins) {
+      const long long nb = B - b0 < wins ? B - b0 : wins;
+      hipLaunchKernelGGL((k_chsum<T, FORM, S>), dim3((unsigned)(slabs * nb)), dim3(256), lds, st, out + b0 * o_ws, o_ws, C,
+                         Wo, NT, TT, slabs, 1.0 / Tn, chsum + b0 * cs_ws, cs_ws);
+    }
   };
   // More channels a block load longer runs of a pixel, fewer make more blocks and longer chunks (a chunk costs its
   // barrier). 64 from four blocks a CU on for images of one chunk (128 windows of 16 x 4 x 1392: 9.8 us, 12.7 with 32,

@@ -178,6 +178,20 @@ def test_channel_sums_chunks(hip, form, dtype, B, H, W, C, k):
     check_case(hip, form, dtype, B, H, W, C, k, 1, k // 2, k // 2, 1, seed=H + W + C, windows=[0, B - 1])
 
 
+def test_channel_sums_many_windows(hip):
+    """More windows than one launch of the sums may have blocks: 1 x 1 px, 4 channels, k = 1, where a sum is the output"""
+    H, rng, B, C = hip, np.random.default_rng(17), (1 << 24) + 3, 4
+    x = rng.standard_normal((B, C), np.float32).astype(np.float16)
+    w, b = rng.standard_normal((1, C)).astype(np.float16), rng.standard_normal(C).astype(np.float16)
+    dx, dw, db = H.DeviceArray.from_host(x), H.DeviceArray.from_host(w), H.DeviceArray.from_host(b)
+    do, ds = H.DeviceArray.zeros((B, C), np.float16), H.DeviceArray.zeros((B, C), np.float32)
+    say("channel sums of", B, "windows")
+    H.check(H.lib().bnh_dwk_f16(dx.ptr, C, 1, 1, C, 1, 1, 0, 0, dw.ptr, db.ptr, 0, do.ptr, C, 1, 1, ds.ptr, C, B, None),
+            "dwk_f16")
+    H.sync()
+    assert np.array_equal(ds.numpy(), do.numpy().astype(np.float32))
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float16])
 @pytest.mark.parametrize("form", ["dwk", "dw3"])
 def test_dw_specials(hip, dtype, form):
