@@ -399,7 +399,7 @@ __global__ __launch_bounds__(256) void k_se_scale(const float *__restrict__ gate
 
 // ------------------------------------------------------------------ MEAN
 // 16 pixels' loads at once, then their sums in order (a load a sum waited on memory for each: 64 px x 1536 channels,
-// one window 16.7 -> 4.3 us)
+// one window 7.5 -> 3.7 us, 128 windows 19.3 -> 8.6, repeated calls; fp16 7.6 -> 3.9, 1000 px x 128 windows 412 -> 72)
 __global__ void k_mean_f32(const float *__restrict__ x, long long x_ws, int P, int C, int ld, float *__restrict__ out,
                            long long o_ws) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x, win = blockIdx.y;
@@ -425,12 +425,12 @@ __global__ void k_mean_f16(const uint16_t *__restrict__ x, long long x_ws, int P
   const uint16_t *xw = x + win * x_ws + c;
   float s = 0.f;
   for (int p = 0; p < P; p += 16) {
-    float v[16];
+    uint16_t v[16];  // widened only in the sums: a conversion beside its load waits for it
 #pragma unroll
-    for (int u = 0; u < 16; u++) v[u] = p + u < P ? (float)hfrom(xw[(long long)(p + u) * ld]) : 0.f;
+    for (int u = 0; u < 16; u++) v[u] = xw[(long long)(p + u < P ? p + u : P - 1) * ld];
 #pragma unroll
     for (int u = 0; u < 16; u++)
-      if (p + u < P) s = s + v[u];
+      if (p + u < P) s = s + (float)hfrom(v[u]);
   }
   out[win * o_ws + c] = s / (float)P;
 }
