@@ -741,6 +741,9 @@ __global__ __launch_bounds__(256) void k_dw_f16v(const h16 *__restrict__ xp, lon
 // Measured against one term a read with a row's bookkeeping between rows: 249 x 63 px x 40 channels (raster order)
 // 217 -> 62 us for one window, 183 -> 82 us for 128; 125 x 32 x 144 43 -> 18 and 80 -> 57; 63 x 16 x 288 (groups)
 // 20 -> 4 and 25 -> 22; fp16 64 x 24 x 288 (row sums) 29 -> 4 and 35 -> 19.
+// ONE: images of one chunk. Their last terms are most or all of them, so those come from registers too (an LDS read a
+// term else), and a tail term loads its own pixels only: with the depthwise conv, 256 windows of 5 x 5 x 1392 in raster
+// order 49.7 -> 35.8 us, 7 x 7 x 816 (k 5) 74.0 -> 65.8, one window of 16 x 4 x 24 fp16 7.8 -> 7.3.
 template <int FORM>
 __host__ __device__ __forceinline__ int cs_terms(int Wo) {  // terms per row
   if (FORM == 0) return Wo / 4 + Wo % 4;
@@ -770,7 +773,7 @@ struct CsPlan {
   static constexpr int U = FORM == 2 ? 8 : 4, TT = U * 192 * 4 / S;
 };
 
-template <typename T, int FORM, int S>
+template <typename T, int FORM, int S, bool ONE>
 __global__ __launch_bounds__(256) void k_chsum(const T *__restrict__ out, long long o_ws, int C, int Wo, int NT, int TT,
                                                int slabs, double rTn, float *__restrict__ chsum, long long cs_ws) {
   extern __shared__ __attribute__((aligned(16))) float tb[];  // [1 or 2][S][TT + 4], 16 floats read past the end
@@ -778,7 +781,7 @@ __global__ __launch_bounds__(256) void k_chsum(const T *__restrict__ out, long l
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const unsigned lb = bnh_xcd_block(blockIdx.x, gridDim.x);  // a window's slabs share pixels' cache lines: one XCD
   const int win = (int)(lb / slabs), c0 = (int)(lb % slabs) * S, ST = TT + 4, per = S * ST;
-  const int items = TT * S4, nch = (NT + TT - 1) / TT;
+  const int items = TT * S4, nch = ONE ? 1 : (NT + TT - 1) / TT;
   const T *o = out + win * o_ws + c0;
   const int Tn = cs_terms<FORM>(Wo), g4 = Wo / 4, np = (Wo % 4) >> 1;
   const bool whole = Wo % 4 == 0;  // rows of whole groups: group t is pixels 4 t .. 4 t + 3 of the image
@@ -803,7 +806,8 @@ __global__ __launch_bounds__(256) void k_chsum(const T *__restrict__ out, long l
       }
       kind[u] = k;
 #pragma unroll
-      for (int i = 0; i < NP; i++) v[u][i].load(p + (long long)(px + (i < k ? i : 0)) * C);
+      for (int i = 0; i < NP; i++)
+        if (!ONE || i < k) v[u][i].load(p + (long long)(px + (i < k ? i : 0)) * C);
     }
   };
   auto write = [&](float *buf, int l, int nl) {
@@ -904,7 +908,20 @@ __global__ __launch_bounds__(256) void k_chsum(const T *__restrict__ out, long l
         read(a, t / 4 + 8);
         add(b);
       }
-      for (; t < n; t++) cs = cs + row[t];
+      if constexpr (ONE) {  // all of a short image's terms are such a rest: from registers, not an LDS read each
+        auto rest = [&](const float4 (&d)[4], int r) {
+#pragma unroll
+          for (int i = 0; i < 16; i++)
+            if (i < r) cs = cs + (i % 4 == 0 ? d[i / 4].x : i % 4 == 1 ? d[i / 4].y : i % 4 == 2 ? d[i / 4].z : d[i / 4].w);
+        };
+        if (n - t >= 16) {
+          read(b, t / 4 + 4);
+          add(a);
+          rest(b, n - t - 16);
+        } else
+          rest(a, n - t);
+      } else
+        for (; t < n; t++) cs = cs + row[t];
     }
     if (ch + 1 < nch) barrier();
   }
@@ -979,8 +996,9 @@ static int chsum_launch(const T *out, long long o_ws, int C, int Ho, int Wo, flo
     const int wins = (1 << 23) / slabs < 1 ? 1 : (1 << 23) / slabs;  // windows a launch: 2^32 threads are too many
     for (long long b0 = 0; b0 < B; b0 += wins) {
       const long long nb = B - b0 < wins ? B - b0 : wins;
-      hipLaunchKernelGGL((k_chsum<T, FORM, S>), dim3((unsigned)(slabs * nb)), dim3(256), lds, st, out + b0 * o_ws, o_ws, C,
-                         Wo, NT, TT, slabs, 1.0 / Tn, chsum + b0 * cs_ws, cs_ws);
+      hipLaunchKernelGGL((NT > TT ? k_chsum<T, FORM, S, false> : k_chsum<T, FORM, S, true>), dim3((unsigned)(slabs * nb)),
+                         dim3(256), lds, st, out + b0 * o_ws, o_ws, C, Wo, NT, TT, slabs, 1.0 / Tn, chsum + b0 * cs_ws,
+                         cs_ws);
     }
   };
   // More channels a block load longer runs of a pixel, fewer make more blocks and longer chunks (a chunk costs its
