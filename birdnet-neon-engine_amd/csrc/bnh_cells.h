@@ -2,26 +2,31 @@
 // their squares as libbnneon's kernels form it (pc_quant_cells_f32, pc_l2norm_f32): 8 fused chains, channel c in chain
 // c % 8 in order of c, combined as ((t0 + t1) + (t2 + t3)) with t_j = chain_j + chain_{j + 4}.
 //
-// A cell is a memory round trip and a serial chain of C / 8 steps, nothing else: 2048 values are fetched at once into
+// A cell is a memory round trip and a serial chain of C / 8 steps, nothing else: 256 NV values are fetched at once into
 // registers (lane l holds values 4 l .. 4 l + 3 of each 256), laid out chain by chain in LDS, and lanes 0..7 read four
 // steps of their chains at a time. Fetched 64 at a time with an LDS read per step, 1280 cells x 1536 took 26.7 us and
 // 192 cells 22.5; the whole head of one window (64 cells, 59,180 int8 prototypes) went from 50.9 to 36.3 us, the fp32
-// head of 3 windows against 5000 from 57.5 to 45.5.
+// head of 3 windows against 5000 from 57.5 to 45.5. NV as C needs it, at most 8: the registers, LDS and code for 2048
+// values cost cells of fewer their occupancy (16,384 cells x 64 to int8 11.0 us fetched 64 at a time, 25.3 with NV 8,
+// 10.3 with NV 1; 8192 x 360 11.4, 16.4, 9.7 with NV 2).
 #ifndef BNH_CELLS_H
 #define BNH_CELLS_H
 #include "bnh_f16.h"
 #include "bnh_num.h"
 
-#define CELL_CH 2048                  // values in registers at a time
-#define CELL_LS (CELL_CH / 8 + 4)     // floats of a chain in LDS
+// NV for cells of C values
+static inline int cell_nv(int C) { return C <= 256 ? 1 : C <= 512 ? 2 : C <= 1024 ? 4 : 8; }
 
+template <int NV>
 struct Cell {
-  float4 v[CELL_CH / 256];
-  // values c0 .. c0 + 2047 of row x, zeros past C; vec: the row is 16-byte (fp16: 8-byte) aligned
+  static constexpr int CH = 256 * NV;    // values in registers at a time
+  static constexpr int LS = CH / 8 + 4;  // floats of a chain in LDS
+  float4 v[NV];
+  // values c0 .. c0 + CH - 1 of row x, zeros past C; vec: the row is 16-byte (fp16: 8-byte) aligned
   template <bool F16>
   BNH_DEV void load(const void *x, int c0, int C, bool vec, int lane) {
 #pragma unroll
-    for (int j = 0; j < CELL_CH / 256; j++) {
+    for (int j = 0; j < NV; j++) {
       const int c = c0 + 256 * j + 4 * lane;
       v[j] = make_float4(0.f, 0.f, 0.f, 0.f);
       if (c >= C) continue;
@@ -39,16 +44,16 @@ struct Cell {
       }
     }
   }
-  // lane l < 8: chain l continued over the n values held; the whole block calls it (s: 8 CELL_LS floats a wave)
+  // lane l < 8: chain l continued over the n values held; the whole block calls it (s: 8 LS floats a wave)
   BNH_DEV float squares(float chain, int n, float *s, int lane) const {
 #pragma unroll
-    for (int j = 0; j < CELL_CH / 256; j++) {
-      float *d = s + 4 * (lane & 1) * CELL_LS + 32 * j + (lane >> 1);
-      d[0] = v[j].x, d[CELL_LS] = v[j].y, d[2 * CELL_LS] = v[j].z, d[3 * CELL_LS] = v[j].w;
+    for (int j = 0; j < NV; j++) {
+      float *d = s + 4 * (lane & 1) * LS + 32 * j + (lane >> 1);
+      d[0] = v[j].x, d[LS] = v[j].y, d[2 * LS] = v[j].z, d[3 * LS] = v[j].w;
     }
     __syncthreads();
     if (lane < 8) {
-      const float *r = s + lane * CELL_LS;
+      const float *r = s + lane * LS;
       const int steps = n / 8;
       int i = 0;
       for (; i + 32 <= steps; i += 32) {

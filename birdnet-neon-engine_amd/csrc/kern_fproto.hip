@@ -38,11 +38,11 @@ struct bnh_fproto {
 // ------------------------------------------------------------------ L2 normalisation of the cells
 // One wave per cell (bnh_cells.h). den = sqrtf(sum) + eps, a = x / den (correctly rounded division); F16: fp16 cells
 // widened, a rounded to fp16 (nearest even). vec, avec: the rows of x and of a are 16-byte (fp16: 8-byte) aligned.
-template <bool F16>
+template <bool F16, int NV>
 __global__ __launch_bounds__(256) void k_l2norm(const void *__restrict__ xv, long long x_ws, int P, int C, int ld,
                                                 float eps, void *__restrict__ av, long long a_ws, long long cells,
                                                 bool vec, bool avec) {
-  __shared__ __attribute__((aligned(16))) float stage[4][8 * CELL_LS];
+  __shared__ __attribute__((aligned(16))) float stage[4][8 * Cell<NV>::LS];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   long long cell = (long long)blockIdx.x * 4 + wv;
   const bool live = cell < cells;
@@ -50,19 +50,20 @@ __global__ __launch_bounds__(256) void k_l2norm(const void *__restrict__ xv, lon
   const long long w = cell / P;
   const int p = (int)(cell - w * P);
   const void *r = (const char *)xv + (w * x_ws + (long long)p * ld) * (F16 ? 2 : 4);
-  Cell x;
+  constexpr int CH = Cell<NV>::CH;
+  Cell<NV> x;
   float chain = 0.f;
-  for (int c0 = 0; c0 < C; c0 += CELL_CH) {
-    x.load<F16>(r, c0, C, vec, lane);
-    chain = x.squares(chain, C - c0 < CELL_CH ? C - c0 : CELL_CH, stage[wv], lane);
+  for (int c0 = 0; c0 < C; c0 += CH) {
+    x.template load<F16>(r, c0, C, vec, lane);
+    chain = x.squares(chain, C - c0 < CH ? C - c0 : CH, stage[wv], lane);
   }
   if (!live) return;
   const float den = cell_norm(chain, lane) + eps;
   const long long at = w * a_ws + (long long)p * C;
-  for (int c0 = 0; c0 < C; c0 += CELL_CH) {
-    if (C > CELL_CH) x.load<F16>(r, c0, C, vec, lane);
+  for (int c0 = 0; c0 < C; c0 += CH) {
+    if (C > CH) x.template load<F16>(r, c0, C, vec, lane);
 #pragma unroll
-    for (int j = 0; j < CELL_CH / 256; j++) {
+    for (int j = 0; j < NV; j++) {
       const int c = c0 + 256 * j + 4 * lane;
       if (c >= C) continue;
       const float4 y = make_float4(x.v[j].x / den, x.v[j].y / den, x.v[j].z / den, x.v[j].w / den);
@@ -468,12 +469,17 @@ int bnh_l2norm_cells(const void *x, long long x_ws, int P, int C, int ld, float 
   const uintptr_t mask = f16 ? 7 : 15;
   const bool vec = ((uintptr_t)x & mask) == 0 && ld % 4 == 0 && (B == 1 || x_ws % 4 == 0);
   const bool avec = ((uintptr_t)a & mask) == 0 && (B == 1 || a_ws % 4 == 0);
-  if (f16)
-    hipLaunchKernelGGL(k_l2norm<true>, dim3((unsigned)bnh_ceil_div(cells, 4)), dim3(256), 0, bnh_stream(stream), x, x_ws,
-                       P, C, ld, eps, a, a_ws, cells, vec, avec);
-  else
-    hipLaunchKernelGGL(k_l2norm<false>, dim3((unsigned)bnh_ceil_div(cells, 4)), dim3(256), 0, bnh_stream(stream), x,
-                       x_ws, P, C, ld, eps, a, a_ws, cells, vec, avec);
+  auto launch = [&](auto nv) {
+    constexpr int NV = decltype(nv)::value;
+    hipLaunchKernelGGL((f16 ? k_l2norm<true, NV> : k_l2norm<false, NV>), dim3((unsigned)bnh_ceil_div(cells, 4)), dim3(256),
+                       0, bnh_stream(stream), x, x_ws, P, C, ld, eps, a, a_ws, cells, vec, avec);
+  };
+  switch (cell_nv(C)) {
+    case 1: launch(std::integral_constant<int, 1>{}); break;
+    case 2: launch(std::integral_constant<int, 2>{}); break;
+    case 4: launch(std::integral_constant<int, 4>{}); break;
+    default: launch(std::integral_constant<int, 8>{});
+  }
   BNH_HIP(hipGetLastError());
   return 0;
 }

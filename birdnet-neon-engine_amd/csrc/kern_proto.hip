@@ -31,12 +31,12 @@ static inline size_t s8p_at(int n, int k, int Kt) {
 // One wave per cell (bnh_cells.h). max |x| (FMAX, NaN-propagating) is order-free: all lanes, then a wave reduction.
 // F16: the cells are fp16 (pc_quant_cells_f16, src/pc_proto_s8.c:14-45: the same sums of the widened values, and
 // codes narrowed with saturation to [-128, 127] without the floor at -127)
-template <bool F16>
+template <bool F16, int NV>
 __global__ __launch_bounds__(256) void k_quant_cells(const void *__restrict__ xv, long long x_ws, int P, int C, int ld,
                                                      float eps, int8_t *__restrict__ qa, long long qa_ws, int Kp,
                                                      float *__restrict__ sx, long long sx_ws, long long cells,
                                                      bool vec) {
-  __shared__ __attribute__((aligned(16))) float stage[4][8 * CELL_LS];
+  __shared__ __attribute__((aligned(16))) float stage[4][8 * Cell<NV>::LS];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   long long cell = (long long)blockIdx.x * 4 + wv;
   const bool live = cell < cells;
@@ -44,15 +44,16 @@ __global__ __launch_bounds__(256) void k_quant_cells(const void *__restrict__ xv
   const long long w = cell / P;
   const int p = (int)(cell - w * P);
   const void *r = (const char *)xv + (w * x_ws + (long long)p * ld) * (F16 ? 2 : 4);
-  Cell x;
+  constexpr int CH = Cell<NV>::CH;
+  Cell<NV> x;
   float chain = 0.f, mx = 0.f;
-  for (int c0 = 0; c0 < C; c0 += CELL_CH) {
-    x.load<F16>(r, c0, C, vec, lane);
+  for (int c0 = 0; c0 < C; c0 += CH) {
+    x.template load<F16>(r, c0, C, vec, lane);
 #pragma unroll
-    for (int j = 0; j < CELL_CH / 256; j++)
+    for (int j = 0; j < NV; j++)
       mx = bnh_fmax(bnh_fmax(bnh_fmax(mx, __builtin_fabsf(x.v[j].x)), __builtin_fabsf(x.v[j].y)),
                     bnh_fmax(__builtin_fabsf(x.v[j].z), __builtin_fabsf(x.v[j].w)));
-    chain = x.squares(chain, C - c0 < CELL_CH ? C - c0 : CELL_CH, stage[wv], lane);
+    chain = x.squares(chain, C - c0 < CH ? C - c0 : CH, stage[wv], lane);
   }
   if (!live) return;
   for (int off = 32; off; off >>= 1) mx = bnh_fmax(mx, __shfl_xor(mx, off));
@@ -61,10 +62,10 @@ __global__ __launch_bounds__(256) void k_quant_cells(const void *__restrict__ xv
   if (lane == 0) sx[w * sx_ws + p] = mx / (127.f * den);
   const float inv = 127.f / mx;
   int8_t *q = qa + w * qa_ws + (long long)p * Kp;
-  for (int c0 = 0; c0 < Kp; c0 += CELL_CH) {
-    if (Kp > CELL_CH) x.load<F16>(r, c0, C, vec, lane);
+  for (int c0 = 0; c0 < Kp; c0 += CH) {
+    if (Kp > CH) x.template load<F16>(r, c0, C, vec, lane);
 #pragma unroll
-    for (int j = 0; j < CELL_CH / 256; j++) {
+    for (int j = 0; j < NV; j++) {
       const int c = c0 + 256 * j + 4 * lane;
       if (c >= Kp) continue;
       const float e[4] = {x.v[j].x, x.v[j].y, x.v[j].z, x.v[j].w};
@@ -534,6 +535,21 @@ __global__ void k_proto_logits(const float *__restrict__ colmax, long long cm_ws
 }
 
 // ================================================================== host side
+template <bool F16>
+static void quant_cells_launch(const void *x, long long x_ws, int P, int C, int ld, float eps, int8_t *qa, long long qa_ws,
+                               int Kp, float *sx, long long sx_ws, long long cells, bool vec, hipStream_t st) {
+#define QCELLS(NV)                                                                                                     \
+  hipLaunchKernelGGL((k_quant_cells<F16, NV>), dim3((unsigned)bnh_ceil_div(cells, 4)), dim3(256), 0, st, x, x_ws, P, C, ld, \
+                     eps, qa, qa_ws, Kp, sx, sx_ws, cells, vec)
+  switch (cell_nv(Kp)) {
+    case 1: QCELLS(1); break;
+    case 2: QCELLS(2); break;
+    case 4: QCELLS(4); break;
+    default: QCELLS(8);
+  }
+#undef QCELLS
+}
+
 extern "C" {
 
 bnh_s8p *bnh_s8p_new(int Np, int Kp, const int8_t *qw, const float *sw) {
@@ -578,8 +594,7 @@ int bnh_quant_cells(const float *x, long long x_ws, int P, int C, int ld, float 
   BNH_REQ(B == 1 || (qa_ws >= (long long)P * Kp && sx_ws >= P && x_ws >= (long long)(P - 1) * ld + C));
   const long long cells = (long long)P * B;
   const bool vec = ((uintptr_t)x & 15) == 0 && ld % 4 == 0 && (B == 1 || x_ws % 4 == 0);
-  hipLaunchKernelGGL(k_quant_cells<false>, dim3((unsigned)bnh_ceil_div(cells, 4)), dim3(256), 0, bnh_stream(stream), x,
-                     x_ws, P, C, ld, eps, qa, qa_ws, Kp, sx, sx_ws, cells, vec);
+  quant_cells_launch<false>(x, x_ws, P, C, ld, eps, qa, qa_ws, Kp, sx, sx_ws, cells, vec, bnh_stream(stream));
   BNH_HIP(hipGetLastError());
   return 0;
 }
@@ -592,8 +607,7 @@ int bnh_quant_cells_f16(const uint16_t *x, long long x_ws, int P, int C, int ld,
   BNH_REQ(B == 1 || (qa_ws >= (long long)P * Kp && sx_ws >= P && x_ws >= (long long)(P - 1) * ld + C));
   const long long cells = (long long)P * B;
   const bool vec = ((uintptr_t)x & 7) == 0 && ld % 4 == 0 && (B == 1 || x_ws % 4 == 0);
-  hipLaunchKernelGGL(k_quant_cells<true>, dim3((unsigned)bnh_ceil_div(cells, 4)), dim3(256), 0, bnh_stream(stream), x,
-                     x_ws, P, C, ld, eps, qa, qa_ws, Kp, sx, sx_ws, cells, vec);
+  quant_cells_launch<true>(x, x_ws, P, C, ld, eps, qa, qa_ws, Kp, sx, sx_ws, cells, vec, bnh_stream(stream));
   BNH_HIP(hipGetLastError());
   return 0;
 }

@@ -49,7 +49,8 @@ def oracle_colmax(kind, a, w, Np):
 
 @pytest.mark.parametrize("fp16", [False, True])
 @pytest.mark.parametrize("P,C,ld", [(64, 1536, 1536), (24, 40, 48), (8, 8, 8), (136, 264, 272), (8, 2048, 2049),
-                                    (9, 2056, 2058), (7, 4360, 4360)])
+                                    (9, 2056, 2058), (7, 4360, 4360), (9, 256, 256), (9, 264, 265), (7, 512, 512),
+                                    (9, 520, 520), (7, 1024, 1026), (10, 1032, 1032)])
 def test_l2norm_cells(hip, fp16, P, C, ld):
     H = hip
     rng = np.random.default_rng(P + C)

@@ -55,7 +55,8 @@ def run_head(H, x, protos, clsw, clsb, nc, eps=1e-5):
 # per-window kernel
 @pytest.mark.parametrize("P,C,N,nc", [(4, 8, 4, 1), (12, 48, 20, 5), (64, 136, 400, 100), (100, 96, 1000, 250),
                                       (64, 256, 1000, 250), (64, 512, 2044, 511), (5, 2048, 12, 3), (9, 2056, 8, 2),
-                                      (4, 4160, 4, 1)])
+                                      (4, 4160, 4, 1), (3, 256, 4, 1), (3, 264, 4, 1), (5, 512, 4, 1), (5, 520, 4, 1),
+                                      (3, 1024, 4, 1), (6, 1032, 4, 1)])  # C at the limits of a cell's registers
 def test_head_small_shapes(hip, P, C, N, nc):
     rng = np.random.default_rng(P + C)
     B = 3
