@@ -301,11 +301,14 @@ struct QdConv {  // the 3 x 3 implicit im2col: A row m = output pixel (m / Wo, m
 // A block owns 128 rows; each wave 32 of them (2 MFMA row tiles) across the 64-channel groups [g0, g1) of its part.
 // CONV: k = 3 C ky + (kx C + c) over the haloed copy (its rows hold the 3 C bytes of kx = 0..2 contiguously), each
 // 16-byte chunk as two 8-byte halves, zero past 9 C.
-// VEC: the weights are the MFMA's first operand and the rows its second, and tile j takes channels 16 q + 4 j + i
-// (q, i = 0..3) of the group: a lane's four tiles then hold 16 neighbouring channels of one row, which it activates
-// (the fp16 SiLU two values at a time from an LDS table) and stores as 16-byte chunks (fp32: the residual chunk added
-// to each), no LDS tile between.
-template <bool CONV, bool VEC>
+// VEC 1 (fp16 out), 2 (fp32 out): the weights are the MFMA's first operand and the rows its second, so a lane holds four neighbouring channels of
+// one row in each tile, which it activates (the fp16 SiLU two values at a time from an LDS table) and stores, no LDS
+// tile between. fp16 outputs of a whole group: tile j takes channels 16 q + 4 j + i (q, i = 0..3), and a lane's four
+// tiles are 16 neighbouring channels, two 16-byte chunks. fp32 outputs (the residual chunk added to each) and partial
+// groups: tile j takes channels 16 j .. 16 j + 15, so that a store's lanes cover 64 bytes of each row and none of them
+// idles in a partial group (131,072 rows x 40 -> 384 fp32 129 -> 45 us against 16 channels a lane, 2048 x 40 -> 16 with
+// SiLU fp32 25.3 -> 6.6, fp16 5.6 -> 3.4; through an LDS tile 62.6, 8.4 and 4.3).
+template <bool CONV, int VEC>
 __global__ __launch_bounds__(256, 4) void k_qd_gemm(const int8_t *__restrict__ a, long long a_ws, int lda,
                                                  const float *__restrict__ rq, long long rq_ws, int per_tensor, int M,
                                                  double rM, long long rows, const int8_t *__restrict__ wt,
@@ -350,8 +353,9 @@ __global__ __launch_bounds__(256, 4) void k_qd_gemm(const int8_t *__restrict__ a
   for (int g = g0; g < g1; g++) {
     const int n0 = 64 * g;
     const int jn = Np - n0 >= 64 ? 4 : (Np - n0) / 16;  // Np % 16 == 0
+    const bool wide = VEC == 1 && jn == 4;
     // weight rows: tile j's channel of this lane is bc + bj j
-    const int bc = VEC ? 16 * ((lane & 15) >> 2) + (lane & 3) : lane & 15, bj = VEC ? 4 : 16;
+    const int bc = wide ? 16 * ((lane & 15) >> 2) + (lane & 3) : lane & 15, bj = wide ? 4 : 16;
     const int8_t *bp = wt + (long long)(n0 + bc) * Kp + kc;
     v4i acc[2][4];
 #pragma unroll
@@ -382,25 +386,24 @@ __global__ __launch_bounds__(256, 4) void k_qd_gemm(const int8_t *__restrict__ a
       }
 #pragma unroll
       for (int j = 0; j < 4; j++)
-        bv[j] = kin && (VEC ? bc >> 4 : j) < jn ? *(const v4i *)(bp + (long long)bj * j * Kp + k0) : (v4i){0, 0, 0, 0};
+        bv[j] = kin && j < jn ? *(const v4i *)(bp + (long long)bj * j * Kp + k0) : (v4i){0, 0, 0, 0};
 #pragma unroll
       for (int t = 0; t < 2; t++)
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-          if constexpr (VEC) acc[t][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bv[j], av[t], acc[t][j], 0, 0, 0);
+          if constexpr (VEC != 0) acc[t][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bv[j], av[t], acc[t][j], 0, 0, 0);
           else if (j < jn) acc[t][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[t], bv[j], acc[t][j], 0, 0, 0);
         }
     }
     // epilogue (tile_row / affine4, src/gemm_s8.c:54-87,143-150)
-    if constexpr (VEC) {
-      if (lane >> 4 >= jn) continue;
-      const int n = n0 + 16 * (lane >> 4);
+    if constexpr (VEC != 0) {
+      const int n = n0 + (wide ? 16 : 4) * (lane >> 4), nj = wide ? 4 : 16;  // tile j: channels n + nj j and three more
       const int lr[2] = {lr0 + (lane & 15), lr0 + 16 + (lane & 15)};
       const bool in[2] = {rowB + lr[0] < rows, rowB + lr[1] < rows};
       const float sav[2] = {s_sa[lr[0]], s_sa[lr[1]]}, zsv[2] = {s_zs[lr[0]], s_zs[lr[1]]};
       auto affine = [&](int t, int j, float v[4]) {
-        const float4 w4 = *(const float4 *)(sw + n + 4 * j), z4 = *(const float4 *)(sws + n + 4 * j);
-        const float4 b4 = *(const float4 *)(bias + n + 4 * j);
+        const int nn = n + nj * j;
+        const float4 w4 = *(const float4 *)(sw + nn), z4 = *(const float4 *)(sws + nn), b4 = *(const float4 *)(bias + nn);
         const float wv[4] = {w4.x, w4.y, w4.z, w4.w}, zv[4] = {z4.x, z4.y, z4.z, z4.w}, bb[4] = {b4.x, b4.y, b4.z, b4.w};
 #pragma unroll
         for (int r = 0; r < 4; r++) {
@@ -408,27 +411,42 @@ __global__ __launch_bounds__(256, 4) void k_qd_gemm(const int8_t *__restrict__ a
           v[r] = __builtin_fmaf(zv[r], zsv[t], __builtin_fmaf(v0, sav[t], bb[r]));
         }
       };
-      if (e.out_f16) {
-        uint32_t h[2][8];
+      if constexpr (VEC == 1) {
+        auto pair = [&](const float *v) {  // two outputs
+          h2 hv = (h2){f2h(v[0]), f2h(v[1])};
+          if (e.act == 1) hv = silu2_lut(hv, s_t01, s_t2);
+          return __builtin_bit_cast(uint32_t, hv);
+        };
+        if (wide) {
+          uint32_t h[2][8];
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+          for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+              float v[4];
+              affine(t, j, v);
+              h[t][2 * j] = pair(v);
+              h[t][2 * j + 1] = pair(v + 2);
+            }
 #pragma unroll
           for (int t = 0; t < 2; t++) {
-            float v[4];
-            affine(t, j, v);
+            if (!in[t]) continue;
+            uint4 *o = (uint4 *)((uint16_t *)e.out + s_o[lr[t]] + n);
+            o[0] = make_uint4(h[t][0], h[t][1], h[t][2], h[t][3]);
+            o[1] = make_uint4(h[t][4], h[t][5], h[t][6], h[t][7]);
+          }
+        } else {
 #pragma unroll
-            for (int r = 0; r < 4; r += 2) {
-              h2 hv = (h2){f2h(v[r]), f2h(v[r + 1])};
-              if (e.act == 1) hv = silu2_lut(hv, s_t01, s_t2);
-              h[t][2 * j + r / 2] = __builtin_bit_cast(uint32_t, hv);
+          for (int j = 0; j < 3; j++) {
+            if (j >= jn) break;
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+              float v[4];
+              affine(t, j, v);
+              const uint2 h = make_uint2(pair(v), pair(v + 2));
+              if (in[t]) *(uint2 *)((uint16_t *)e.out + s_o[lr[t]] + n + 16 * j) = h;
             }
           }
-#pragma unroll
-        for (int t = 0; t < 2; t++) {
-          if (!in[t]) continue;
-          uint4 *o = (uint4 *)((uint16_t *)e.out + s_o[lr[t]] + n);
-          o[0] = make_uint4(h[t][0], h[t][1], h[t][2], h[t][3]);
-          o[1] = make_uint4(h[t][4], h[t][5], h[t][6], h[t][7]);
         }
       } else {  // the residual chunks loaded before any store (out and res may alias)
         float4 rv[2][4];
@@ -436,9 +454,11 @@ __global__ __launch_bounds__(256, 4) void k_qd_gemm(const int8_t *__restrict__ a
         for (int t = 0; t < 2; t++)
 #pragma unroll
           for (int j = 0; j < 4; j++)
-            rv[t][j] = e.res && in[t] ? *(const float4 *)(e.res + s_r[lr[t]] + n + 4 * j) : make_float4(0.f, 0.f, 0.f, 0.f);
+            rv[t][j] = e.res && in[t] && j < jn ? *(const float4 *)(e.res + s_r[lr[t]] + n + 16 * j)
+                                                : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+        for (int j = 0; j < 4; j++) {
+          if (j >= jn) break;
 #pragma unroll
           for (int t = 0; t < 2; t++) {
             float y[4];
@@ -454,8 +474,9 @@ __global__ __launch_bounds__(256, 4) void k_qd_gemm(const int8_t *__restrict__ a
               y[2] = y[2] + rv[t][j].z;
               y[3] = y[3] + rv[t][j].w;
             }
-            if (in[t]) *(float4 *)((float *)e.out + s_o[lr[t]] + n + 4 * j) = make_float4(y[0], y[1], y[2], y[3]);
+            if (in[t]) *(float4 *)((float *)e.out + s_o[lr[t]] + n + 16 * j) = make_float4(y[0], y[1], y[2], y[3]);
           }
+        }
       }
       continue;
     }
@@ -838,11 +859,13 @@ static int qd_gemm_launch(bool conv, const int8_t *a, long long a_ws, int lda, c
   hipLaunchKernelGGL((k_qd_gemm<CV, VC>), grid, dim3(256), 0, bnh_stream(stream), a, a_ws, lda, rq, rq_ws, per_tensor, \
                      M, 1.0 / M, rows, W->w, W->scale, W->swsum, W->bias, W->Kp, W->Np, gsplit, d, cv)
   if (conv) {
-    if (vec) QDG(true, true);
-    else QDG(true, false);
+    if (!vec) QDG(true, 0);
+    else if (e->out_f16) QDG(true, 1);
+    else QDG(true, 2);
   } else {
-    if (vec) QDG(false, true);
-    else QDG(false, false);
+    if (!vec) QDG(false, 0);
+    else if (e->out_f16) QDG(false, 1);
+    else QDG(false, 2);
   }
 #undef QDG
   BNH_HIP(hipGetLastError());

@@ -142,7 +142,8 @@ def run_gemm(hip, a, rq, W, act, out16, M, opad=0, ow=0, res=None, per_tensor=Fa
     return do.numpy()[:, :rows * ldo].reshape(B, rows, ldo), ldo
 
 
-@pytest.mark.parametrize("M,K,N", [(1, 64, 16), (37, 40, 48), (130, 136, 80), (300, 1152, 144), (64, 24, 272)])
+@pytest.mark.parametrize("M,K,N", [(1, 64, 16), (37, 40, 48), (130, 136, 80), (300, 1152, 144), (64, 24, 272), (70, 40, 32),
+                                   (257, 72, 96), (129, 16, 64)])
 @pytest.mark.parametrize("form", ["f32", "f32_silu", "f32_relu_res", "f16", "f16_silu"])
 def test_qd_gemm_epilogues(hip, M, K, N, form):
     rng = np.random.default_rng(M * 7 + K + N)
