@@ -265,6 +265,11 @@ static void ff_launch(const float *a, long long a_ws, int P, const bnh_fproto *W
   double least = 0;
   for (const auto &p : plan) {
     const long long blocks = B * bnh_ceil_div(W->Np, 16 * p.tn * (4 / p.wc));
+    // with four and more blocks a CU the registers of 6 and 8 tiles a wave leave too few waves to cover a block's start:
+    // 64 windows of 64 cells against 20,000 fp32 prototypes, 2 x 2 tiles a wave for 4 x 2, K 64 251 -> 177 us, 200 441 -> 360,
+    // 20 windows of K 1536 718 -> 666; fp16-stored ones, whose operands are half as wide, below K 256 only. What is left
+    // to the vector unit's kernel before: K 64 160 us, K 8 73 against 122.
+    if (blocks >= 1024 && (WH ? p.tc * p.tn == 8 && W->K <= 256 : p.tc * p.tn > 4)) continue;
     const double cost = (double)bnh_ceil_div(blocks, 256) * bnh_ceil_div(P, 16 * p.tc * p.wc) * (p.tc * p.tn + 0.5);
     if (least == 0 || cost < least) least = cost, best = {p.tc, p.wc, p.tn};
   }
