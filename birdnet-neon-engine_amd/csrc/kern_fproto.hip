@@ -254,7 +254,7 @@ __global__ __launch_bounds__(256) void k_colmax_f32(const float *__restrict__ a,
 
 template <bool WH>
 static void ff_launch(const float *a, long long a_ws, int P, const bnh_fproto *W, float *colmax, long long cm_ws, int B,
-                      hipStream_t st) {
+                      bool over, hipStream_t st) {
   // The split with the least work on the fullest CU: its blocks there times the passes over the cells times a wave's
   // step (TC TN matrix instructions and about half of one for its operands). 64 cells x 1536 against 5000 prototypes:
   // 3 windows 4 cell tiles a wave 38 us, 2 by 2 waves 39, 1 by 4 waves 47 (281 us on the vector unit); one window 34, 23
@@ -264,6 +264,10 @@ static void ff_launch(const float *a, long long a_ws, int P, const bnh_fproto *W
                                                     {2, 1, 1}, {3, 2, 1}, {2, 2, 1}, {1, 2, 1}, {1, 4, 1}};
   double least = 0;
   for (const auto &p : plan) {
+    if (over) {  // the first of the list: one block a window
+      best = {p.tc, p.wc, p.tn};
+      break;
+    }
     const long long blocks = B * bnh_ceil_div(W->Np, 16 * p.tn * (4 / p.wc));
     // with four and more blocks a CU the registers of 6 and 8 tiles a wave leave too few waves to cover a block's start:
     // 64 windows of 64 cells against 20,000 fp32 prototypes, 2 x 2 tiles a wave for 4 x 2, K 64 251 -> 177 us, 200 441 -> 360,
@@ -501,14 +505,18 @@ int bnh_fproto_colmax(const void *a, long long a_ws, int P, const bnh_fproto *W,
     hipLaunchKernelGGL(k_colmax_f16, dim3((unsigned)blocks), dim3(256), 0, bnh_stream(stream), (const uint16_t *)a, a_ws,
                        P, W->K, (const uint16_t *)W->w, W->Npt, W->Np, W->bs, W->nblk, colmax, cm_ws, B);
   } else {
+    // maxima over their cells: with one block a window, which has read all of them when it has passed its last barrier
+    const bool over = bnh_overlap(bnh_windows(colmax, cm_ws, W->Np),
+                                  bnh_windows((const float *)a, a_ws, (long long)P * W->K), B);
+    BNH_REQ(!over || W->Np <= 128);
     // windows per launch such that its tiles of 16 prototypes stay under 2^23 (a grid dimension is limited in threads)
     const long long fit = (1LL << 23) / bnh_ceil_div(W->Np, 16);
     const int most = fit < 1 ? 1 : fit > B ? B : (int)fit;
     for (int b0 = 0; b0 < B; b0 += most) {
       const int nb = B - b0 < most ? B - b0 : most;
       const float *ab = (const float *)a + b0 * a_ws;
-      if (W->kind == 1) ff_launch<true>(ab, a_ws, P, W, colmax + b0 * cm_ws, cm_ws, nb, bnh_stream(stream));
-      else ff_launch<false>(ab, a_ws, P, W, colmax + b0 * cm_ws, cm_ws, nb, bnh_stream(stream));
+      if (W->kind == 1) ff_launch<true>(ab, a_ws, P, W, colmax + b0 * cm_ws, cm_ws, nb, over, bnh_stream(stream));
+      else ff_launch<false>(ab, a_ws, P, W, colmax + b0 * cm_ws, cm_ws, nb, over, bnh_stream(stream));
       BNH_HIP(hipGetLastError());
     }
   }

@@ -134,6 +134,28 @@ def test_colmax_f32_splits(hip, P, K, N, B):
             assert same(got[b], ref), (kind, b, np.argwhere(got[b] != ref)[:4])
 
 
+@pytest.mark.parametrize("kind", ["f32", "f32h"])
+@pytest.mark.parametrize("B,P,K,N", [(1, 64, 64, 128), (9, 40, 136, 104), (3, 100, 32, 16)])
+def test_colmax_over_its_cells(hip, kind, B, P, K, N):
+    """Up to 128 maxima in the memory of their window's cells: one block a window reads them all before it stores; more
+    are refused"""
+    H, rng = hip, np.random.default_rng(P + K + N)
+    w, Np = pack(kind, rng.standard_normal((N, K)).astype(f32))
+    Wd = H.FProto(KIND[kind], Np, K, w)
+    cells = rng.standard_normal((B, P * K)).astype(f32)
+    da = H.DeviceArray.from_host(cells)
+    say("colmax over its cells", kind, B, P, K, N)
+    H.check(H.lib().bnh_fproto_colmax(da.ptr, P * K, P, Wd.h, da.ptr, P * K, B, None), "colmax")
+    H.sync()
+    got = da.numpy()
+    for b in range(B):
+        assert same(got[b, :Np], oracle_colmax(kind, cells[b].reshape(P, K), w, Np)), b
+    assert np.array_equal(got[:, Np:], cells[:, Np:])
+    w2, Np2 = pack(kind, rng.standard_normal((136, K)).astype(f32))
+    W2 = H.FProto(KIND[kind], Np2, K, w2)
+    assert H.lib().bnh_fproto_colmax(da.ptr, P * K, P, W2.h, da.ptr, P * K, B, None) != 0
+
+
 @pytest.mark.parametrize("kind", ["f32", "f32h", "f16"])
 def test_colmax_orders_and_specials(hip, kind):
     """rows whose chains the reference's order decides (absorption at 2^24 / fp16 2048, a fused product on -1),
