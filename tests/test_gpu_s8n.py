@@ -157,7 +157,9 @@ def test_quant_rows_gate(hip):
 
 
 def pw_case(hip, B, H_, W_, K, N, act, opad=0, res=False, lda_extra=0, seed=0, gate=False, ldo_extra=8, rpad=0,
-            wins=None, edge=False):
+            wins=None, edge=False, two=False):
+    """one bnh_pw_s8, or (two) its parts as callers of their own may run them: the halo zeroed, bnh_s8n_quant_rows,
+    bnh_s8n_gemm, which is the two-launch form whatever the size"""
     H = hip
     rng = np.random.default_rng(seed)
     M = H_ * W_
@@ -197,8 +199,15 @@ def pw_case(hip, B, H_, W_, K, N, act, opad=0, res=False, lda_extra=0, seed=0, g
     e = H.epi32(dout, ldo, act=act, ow=W_ if opad else 0, opad=opad, res=dres,
                 ldr=Np if res else 0, rpad=rpad, rw=W_ if rpad else 0, out_ws=out_rows * ldo, res_ws=rrows * Np)
     say(f"pw_s8 B{B} {H_}x{W_} K{K} N{N} act{act} opad{opad} res{res} gate{gate}")
-    H.check(H.lib().bnh_pw_s8(dx.ptr, M * lda, lda, M, H.ptr(dg), K if gate else 0, dq.ptr, M4 * Kp,
-                              dsa.ptr, M4, dza.ptr, M4, B, Wt.h, e, None), "pw_s8")
+    if two:
+        if opad:
+            H.check(H.lib().bnh_zero_halo(dout.ptr, out_rows * ldo, H_, W_, ldo, opad, 4, B, None), "zero_halo")
+        H.check(H.lib().bnh_s8n_quant_rows(dx.ptr, M * lda, lda, M, K, Kp, H.ptr(dg), K if gate else 0, dq.ptr, M4 * Kp,
+                                           dsa.ptr, M4, dza.ptr, M4, B, None), "quant_rows")
+        H.check(H.lib().bnh_s8n_gemm(dq.ptr, M4 * Kp, dsa.ptr, M4, dza.ptr, M4, M, B, Wt.h, e, None), "gemm")
+    else:
+        H.check(H.lib().bnh_pw_s8(dx.ptr, M * lda, lda, M, H.ptr(dg), K if gate else 0, dq.ptr, M4 * Kp,
+                                  dsa.ptr, M4, dza.ptr, M4, B, Wt.h, e, None), "pw_s8")
     H.sync()
     out = dout.numpy().reshape(B, out_rows, ldo)
     q = dq.numpy().reshape(B, M4, Kp)
@@ -226,10 +235,13 @@ def test_pw_s8_config0_shape(hip):
 
 def test_pw_s8_large_k_tile_kernel(hip):
     """Kp >= 256 with rows for 1024+ tiles: the LDS-staged tile GEMM (k_s8n_gemm_lds). 128 x 256 tiles at config 0's
-    1152 -> 256 (86 windows); 256 x 128 tiles with a residual from a zero-haloed buffer into a haloed output
-    (N = 100); ldo odd (values stored one by one) with a gate; windows at both ends and the middle checked"""
+    1152 -> 256 (86 windows); 256 x 128 tiles after a quantization of its own, with a residual from a zero-haloed buffer
+    into a haloed output (N = 100) and without (the same sizes in one bnh_pw_s8 quantise their rows beside the products);
+    ldo odd (values stored one by one) with a gate; windows at both ends and the middle checked"""
     assert pw_case(hip, 86, 24, 64, 1152, 256, 1, seed=41, wins=(0, 43, 85))
-    assert pw_case(hip, 128, 32, 64, 320, 100, 2, opad=1, res=True, rpad=1, seed=42, wins=(0, 77, 127))
+    for two in (True, False):
+        assert pw_case(hip, 128, 32, 64, 320, 100, 2, opad=1, res=True, rpad=1, seed=42, wins=(0, 77, 127), two=two)
+    assert pw_case(hip, 128, 32, 64, 320, 100, 1, seed=44, wins=(0, 127), two=True)
     assert pw_case(hip, 86, 24, 64, 256, 200, 0, seed=43, gate=True, ldo_extra=1, wins=(0, 85))
 
 
@@ -239,13 +251,14 @@ def test_pw_s8_residual_halo_gate(hip):
     assert pw_case(hip, 1, 1, 1, 24, 8, 0, seed=11)   # a single row (GEMV-like)
 
 
-def test_pw_s8_residual_quads_split_groups(hip):
-    """The residual epilogue's 16-byte-quad form (ldo and ldr multiples of 4) with three 64-channel groups, the last
+@pytest.mark.parametrize("two", [True, False])
+def test_pw_s8_residual_quads_split_groups(hip, two):
+    """Two launches and one. Two: the residual epilogue's 16-byte-quad form (ldo and ldr multiples of 4) with three 64-channel groups, the last
     one partial (N = 136), the groups split over blocks (few rows: gsplit > 1), and zero-haloed residual and output
     buffers (rpad 1, opad 1), as well as an unhaloed residual into a haloed output."""
-    assert pw_case(hip, 3, 7, 9, 48, 136, 1, opad=1, res=True, rpad=1, seed=14)
-    assert pw_case(hip, 2, 6, 11, 96, 136, 0, opad=2, res=True, rpad=0, seed=15)
-    assert pw_case(hip, 2, 5, 5, 232, 200, 2, opad=0, res=True, rpad=2, seed=16, gate=True)
+    assert pw_case(hip, 3, 7, 9, 48, 136, 1, opad=1, res=True, rpad=1, seed=14, two=two)
+    assert pw_case(hip, 2, 6, 11, 96, 136, 0, opad=2, res=True, rpad=0, seed=15, two=two)
+    assert pw_case(hip, 2, 5, 5, 232, 200, 2, opad=0, res=True, rpad=2, seed=16, gate=True, two=two)
 
 
 def test_pw_s8_unaligned_output_rows(hip):
@@ -257,9 +270,11 @@ def test_pw_s8_unaligned_output_rows(hip):
 
 @pytest.mark.parametrize("K", [48, 49, 52, 64, 65, 128])
 def test_pw_s8_whole_k_steps(hip, K):
-    """Rows that end exactly with a 64-wide K step (Kp 64, 128) and beside it, with and without a residual"""
-    assert pw_case(hip, 2, 6, 11, K, 96, 1, seed=50 + K)
-    assert pw_case(hip, 2, 6, 11, K, 24, 0, res=True, seed=60 + K)
+    """Rows that end exactly with a 64-wide K step (Kp 64, 128) and beside it, with and without a residual, in two
+    launches (whatever K) and in one (K a multiple of 4)"""
+    for two in (True, False):
+        assert pw_case(hip, 2, 6, 11, K, 96, 1, seed=50 + K, two=two)
+        assert pw_case(hip, 2, 6, 11, K, 24, 0, res=True, seed=60 + K, two=two)
 
 
 @pytest.mark.parametrize("K", [4, 60, 128, 132, 256, 260, 512, 516, 1020, 1536, 1540])
