@@ -4,7 +4,7 @@ tail form (K % 4, K % 8, K % 16), the int8 GEMM's fp32 FMA epilogue in all its o
 and without a zero halo, fp32 + silu_f32_a / ReLU / residual), partial K steps and channel groups, the 3 x 3
 implicit-im2col conv at both strides and odd sizes, the SED heads, the fp16-weight SE gate, the generalised mean
 (within one unit in the last place of the C library's powf, which it does not restate) and the scalar functions.
-Inputs are finite (NaN inputs are outside what these kernels are compared on)."""
+Inputs are finite but in the row quantisers' test of special values."""
 import ctypes as ct
 
 import numpy as np
@@ -117,6 +117,52 @@ def test_quant_rows_f16(hip, K, gated):
         ra, rr = O.qd_quant_rows(x[i], K, None if g is None else g[i])
         assert np.array_equal(a[i, :M * Kp].reshape(M, Kp), ra), i
         assert same(rq[i].reshape(M, 2), rr), i
+
+
+def special_rows(rng, K, f16):
+    """[M][K]: NaNs in the first, a middle and the last value of rows between ordinary ones, infinities, zeros of either
+    sign, values at the end of the fp16 range; and the rows whose codes come of a NaN made by an operation (its sign is
+    the processor's)."""
+    big, M = 65504.0 if f16 else 3e38, 24
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    for r, c in ((2, 0), (5, K - 1), (8, K // 2), (9, min(K - 1, 7)), (11, K - 8)):
+        x[r, c] = np.nan
+    x[13, K // 3], x[14, K - 1], x[15, 0] = np.inf, -np.inf, np.inf
+    x[16], x[17], x[18] = -0.0, 0.0, np.where(np.arange(K) % 2, 0.0, -0.0)
+    x[19] *= big / 8
+    x[20], x[21, 0], x[22] = big, -big, -big
+    return x.astype(np.float16 if f16 else np.float32), [13, 14, 15]
+
+
+@pytest.mark.parametrize("K", [8, 16, 24, 32, 56, 64, 128, 200, 256, 512, 520, 1024, 2048])
+@pytest.mark.parametrize("form", ["f32", "f16", "f16 gated"])
+def test_quant_rows_specials(hip, K, form):
+    """NaNs, infinities (with a gate also infinity x 0), signed zeros and the largest values beside ordinary rows, for each
+    number of lanes a row takes: the multi-row vector kernel's codes, scales and zero points against the kernel of one
+    wavefront a row (rows not 16-byte aligned) and the oracle"""
+    H, rng, f16 = hip, np.random.default_rng(K), form != "f32"
+    x, made = special_rows(rng, K, f16)
+    M, Kp, g = len(x), (K + 15) // 16 * 16, None
+    if form == "f16 gated":
+        g = rng.uniform(0.25, 1, K).astype(np.float16)
+        g[K // 3], g[0] = 0.0, 0.5
+    say("quant_rows specials", form, K)
+    got = []
+    for pad in (8, 5):
+        xs = np.zeros((M, K + pad), x.dtype)
+        xs[:, :K] = x
+        dx, da = H.DeviceArray.from_host(xs), H.DeviceArray.from_host(np.full((M, Kp), 99, np.int8))
+        dr, dg = H.DeviceArray.zeros((M, 2), np.float32), None if g is None else H.DeviceArray.from_host(g)
+        H.check(H.lib().bnh_qd_quant_rows(dx.ptr, int(f16), 0, K + pad, M, K, H.ptr(dg), 0, da.ptr, 0, dr.ptr, 0, 1, None),
+                "quant")
+        H.sync()
+        got.append((da.numpy(), dr.numpy()))
+    assert np.array_equal(got[0][0], got[1][0]) and same(got[0][1], got[1][1])
+    with np.errstate(all="ignore"):
+        ra, rr = O.qd_quant_rows(x, K, g)
+    rows = [r for r in range(M) if r not in made]
+    assert same(got[0][1][:, 0], rr[:, 0]) and same(got[0][1][rows], rr[rows])
+    assert np.array_equal(got[0][0][rows], ra[rows]), np.argwhere(got[0][0][rows] != ra[rows])[:4]
 
 
 def run_gemm(hip, a, rq, W, act, out16, M, opad=0, ow=0, res=None, per_tensor=False):
