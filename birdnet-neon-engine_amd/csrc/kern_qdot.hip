@@ -301,13 +301,13 @@ struct QdConv {  // the 3 x 3 implicit im2col: A row m = output pixel (m / Wo, m
 // A block owns 128 rows; each wave 32 of them (2 MFMA row tiles) across the 64-channel groups [g0, g1) of its part.
 // CONV: k = 3 C ky + (kx C + c) over the haloed copy (its rows hold the 3 C bytes of kx = 0..2 contiguously), each
 // 16-byte chunk as two 8-byte halves, zero past 9 C.
-// VEC 1 (fp16 out), 2 (fp32 out): the weights are the MFMA's first operand and the rows its second, so a lane holds four neighbouring channels of
-// one row in each tile, which it activates (the fp16 SiLU two values at a time from an LDS table) and stores, no LDS
-// tile between. fp16 outputs of a whole group: tile j takes channels 16 q + 4 j + i (q, i = 0..3), and a lane's four
-// tiles are 16 neighbouring channels, two 16-byte chunks. fp32 outputs (the residual chunk added to each) and partial
-// groups: tile j takes channels 16 j .. 16 j + 15, so that a store's lanes cover 64 bytes of each row and none of them
-// idles in a partial group (131,072 rows x 40 -> 384 fp32 129 -> 45 us against 16 channels a lane, 2048 x 40 -> 16 with
-// SiLU fp32 25.3 -> 6.6, fp16 5.6 -> 3.4; through an LDS tile 62.6, 8.4 and 4.3).
+// VEC 1 (fp16 out), 2 (fp32 out): the weights are the MFMA's first operand and the rows its second, so a lane holds four
+// neighbouring channels of one row in each tile, which it activates (the fp16 SiLU two values at a time from an LDS
+// table) and stores, no LDS tile between. fp16 outputs of a whole group: tile j takes channels 16 q + 4 j + i (q, i =
+// 0..3), and a lane's four tiles are 16 neighbouring channels, two 16-byte chunks. fp32 outputs (the residual chunk added
+// to each) and partial groups: tile j takes channels 16 j .. 16 j + 15, so that a store's lanes cover 64 bytes of each row
+// and none of them idles in a partial group (131,072 rows x 40 -> 384 fp32 129 -> 45 us against 16 channels a lane, 2048 x
+// 40 -> 16 with SiLU fp32 25.3 -> 6.6, fp16 5.6 -> 3.4; through an LDS tile 62.6, 8.4 and 4.3).
 template <bool CONV, int VEC>
 __global__ __launch_bounds__(256, 4) void k_qd_gemm(const int8_t *__restrict__ a, long long a_ws, int lda,
                                                  const float *__restrict__ rq, long long rq_ws, int per_tensor, int M,
