@@ -469,7 +469,7 @@ __global__ __launch_bounds__(256, 4) void k_s8n_gemm(const int8_t *__restrict__ 
 // one row read, one weight read and the epilogue. The weights are the MFMA's first operand and the rows its second: a
 // lane then holds four neighbouring channels of one row, so residuals are read and outputs stored as 16-byte quads.
 // 16 rows a block: all their loads are in flight at once and five or more blocks share a CU (64 and 32 rows a block
-// read them in several round trips: 63 x 16 px x 40 windows, 288 -> 48, 33.7 and 29.8 us against 23.1).
+// read them in several round trips: 63 x 16 px x 40 windows, 288 -> 48, 33.7 and 29.8 us against 22.7).
 struct QRows {  // the rows to quantise, and where a caller's workspace keeps them (q NULL: nowhere)
   const float *x;
   long long x_ws;
@@ -643,8 +643,8 @@ BNH_DEV void qgemm_rows(const QRows &q, const QGemm &p, long long rowB, long lon
 
 // Many rows: a block owns 16 rows and every channel; each wave multiplies its share of the 16-channel tiles, two at a
 // time, the weights of four 64-byte K steps loaded together. With the SE gate and residual, 63 x 16 px: 288 -> 48,
-// 40 windows 28.9 -> 23.1 us (two launches -> this), 256 windows 138 -> 125 us; 32 x 8 px, 288 -> 96, 40 windows
-// 17.2 -> 10.1 us.
+// 40 windows 28.6 -> 22.7 us (two launches -> this), 256 windows 138 -> 121 us; 32 x 8 px, 288 -> 96, 40 windows
+// 17.0 -> 10.5 us.
 template <int L, int QC, int NR, bool RES>
 __global__ __launch_bounds__(256, 4) void k_s8n_qgemm(QRows q, QGemm p) {
   constexpr int R = 16, CT = 2, KC = 4;
@@ -699,8 +699,8 @@ __global__ __launch_bounds__(256, 4) void k_s8n_qgemm(QRows q, QGemm p) {
 
 // Few rows: a block owns 16 rows and 32 channels (parts blocks quantise the same rows), its waves a quarter of the K
 // steps each, all their weights loaded before the rows are quantised; the waves' int32 sums meet in LDS, in any order
-// the same. Kp <= 64 * 4 * KS. One window, two launches -> this: 63 x 16 px, 288 -> 48 13.8 -> 7.0 us; 16 x 4 px,
-// 1392 -> 232 24 -> 13.5 us; 1536 -> 14,795 over one row 19 -> 14.8 us.
+// the same. Kp <= 64 * 4 * KS. One window, two launches -> this: 63 x 16 px, 288 -> 48 13.4 -> 6.6 us; 16 x 4 px,
+// 1392 -> 232 24 -> 13.0 us; 1536 -> 14,795 over one row 18.3 -> 13.7 us.
 template <int L, int QC, int NR, int KS, bool RES>
 __global__ __launch_bounds__(256) void k_s8n_qgemm16(QRows q, QGemm p, int parts) {
   constexpr int R = 16, CT = 2;

@@ -9,6 +9,14 @@
  * Return value: 0 on success; -1 with bnh_last_error() (thread-local, <= 511 bytes) describing the failure.
  * Shapes are checked on the host before any launch; nothing here allocates device memory except the *_new
  * constructors and bnh_malloc.
+ *
+ * An output shares no memory with an input of the same call unless an entry's comment says so, but: a residual may lie where the output does (the same
+ * rows and strides); bnh_pw_s8's output may lie over its rows and gate; bnh_gemm_f32's with Np <= 64 over its rows (each
+ * output row on its own input row, or windows of at most 64 rows) or, in windows of at most 64 rows, over its gate;
+ * bnh_wino_f16's over its input for W <= 32 (the same rows and strides, opad 1); bnh_gemv's over its input for N <= 32 (the
+ * same stride); bnh_fproto_colmax's over its own window's cells for Np <= 128 (kinds 0, 1; more are refused) or 256 (kind
+ * 2); bnh_l2norm_cells' where its cells lie (the same rows and strides). Windows or columns side by side in one buffer
+ * share nothing.
  */
 #ifndef BNNEON_HIP_H
 #define BNNEON_HIP_H
@@ -124,7 +132,8 @@ int bnh_proto_logits(const float *colmax, long long cm_ws, const float *clsw, co
  * (src/rt_ops_f16.c:227-250). Prototypes from the package tensor, K % 8 == 0 and Np % 8 == 0:
  *   kind 0: fp32 panels [Np/8][K][8] (fpack, Kp = K), kind 1: fp16 panels [Np/8][K][8] (PROTO_F32H),
  *   kind 2: fp16 panels [Np/16][K][16] then a tail panel [K][8] when Np % 16 == 8 (hpack, Kp = K);
- * repacked once into k-major rows in HBM. */
+ * repacked once in HBM: kinds 0 and 1 into tiles of 16 prototypes x 16 k in the matrix instruction's operand order, kind
+ * 2 into k-major rows. */
 typedef struct bnh_fproto bnh_fproto;
 bnh_fproto *bnh_fproto_new(int kind, int Np, int K, const void *w);
 void bnh_fproto_free(bnh_fproto *W);
